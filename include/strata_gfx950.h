@@ -184,6 +184,12 @@ int strata_route_tiles(const uint32_t* idx, int64_t pairs, int64_t k, int64_t ex
 int strata_rows_to_f16(const void* a, int64_t rows, int64_t cols, int a_dtype, void* out, uint32_t* row_max,
                        void* stream);
 
+/* strata_rows_to_f16 with each run of 32 scaled values summed as well: sums float16 (rows, cols / 256, 16), a step of
+ * 256 columns its 8 runs' sums over 32 rounded to float16, then what the rounding left. cols whole steps of 256. What
+ * the tile kernels of the types with mins (Q4_K, Q5_K) multiply those mins by. */
+int strata_rows_to_f16_sums(const void* a, int64_t rows, int64_t cols, int a_dtype, void* out, uint32_t* row_max,
+                            void* sums, void* stream);
+
 /* The inverse of strata_rows_to_f16's scaling, for products of the scaled rows: out[r, c] = c[r, c] * 2^e(r) rounded
  * once to out_dtype (BF16, F16 or F32), e(r) from row_max[r] as strata_rows_to_f16 set it; c float32 (rows, cols),
  * out (rows, cols), at most 65535 rows. No counterpart in the reference, which multiplies a prompt chunk's
@@ -238,6 +244,19 @@ int strata_prompt_down(int kind, const void* blocks, int64_t experts, int64_t ro
                        const uint32_t* h_max, const uint32_t* tile_expert, int64_t n_tiles, int64_t tile,
                        const uint32_t* slot_pair, const uint32_t* idx, int64_t pairs, void* y, int y_dtype,
                        void* stream);
+
+/* The two calls above for every type here, with rows of whole 256-weight steps or, in the types with blocks of 32 or
+ * 64 weights, of whole 64-weight run pairs (cols a multiple of 64); else STRATA_ERR_SHAPE. The types with a min to
+ * each run (Q4_K, Q5_K) take rows scaled by strata_rows_to_f16_sums and its sums (x_sum, h_sum; else NULL, as the
+ * other types'). A row of such a type holding an infinity gives NaN. */
+int strata_tiles_gate_up_swiglu(int kind, const void* gate, const void* up, int64_t experts, int64_t rows,
+                                int64_t cols, const void* x, const uint32_t* x_max, const void* x_sum,
+                                const uint32_t* token, const uint32_t* tile_expert, int64_t n_tiles, int64_t tile,
+                                void* h, int h_dtype, void* stream);
+int strata_tiles_down(int kind, const void* blocks, int64_t experts, int64_t rows, int64_t cols, const void* h,
+                      const uint32_t* h_max, const void* h_sum, const uint32_t* tile_expert, int64_t n_tiles,
+                      int64_t tile, const uint32_t* slot_pair, const uint32_t* idx, int64_t pairs, void* y,
+                      int y_dtype, void* stream);
 
 /* out[t, r] = W[r, :] . x[t, :] for a float16 W (rows x cols, row-major) and `tokens` rows of x
  * (STRATA_F16 or STRATA_F32); out (tokens, rows) float32. cols must be a multiple of 8. The router's

@@ -708,18 +708,40 @@ def tile_matmul(blocks: torch.Tensor, kind: str, shape: tuple, a: torch.Tensor, 
     return out
 
 
-PROMPT_KINDS = ("IQ3_S", "IQ3_XXS", "Q2_0")  # the kinds of the fused prompt kernels (rows of whole 256-weight steps)
+MIN_KINDS = ("Q4_K", "Q5_K")  # types with a min to each run, whose tile kernels take the runs' sums of activations
 
 
 def _prompt_fused(lin, dtype: torch.dtype) -> bool:
-    return lin.kind in PROMPT_KINDS and lin.input_dims % 256 == 0 and dtype in (torch.float16, torch.bfloat16)
+    """Stacks the fused tile kernels take: 16-bit activations, rows of whole 256-weight steps, or of whole 64-weight
+    run pairs in the types with smaller blocks; a matrix below 4 GiB (32-bit row offsets)."""
+    per_block = {**BLOCK, **DENSE}[lin.kind][0]
+    return (dtype in (torch.float16, torch.bfloat16) and lin.kind not in NO_GRID
+            and lin.input_dims % (64 if per_block < 256 else 256) == 0
+            and lin.output_dims * lin.row_bytes < 1 << 32)
+
+
+def _tile_rows(a: torch.Tensor, kind: str) -> tuple:
+    """Activations as the fused tile kernels of `kind` take them: (float16 rows, their largest magnitudes or None, the
+    runs' sums or None). float16 rows go as they are, bfloat16 ones scaled by a power of two each (rows_to_f16); the
+    types with mins take scaled rows of either, with the sums of each run of 32 values."""
+    a = a.reshape(-1, a.shape[-1]).contiguous()
+    if kind not in MIN_KINDS:
+        return (*rows_to_f16(a), None) if a.dtype == torch.bfloat16 else (a, None, None)
+    rows, cols = a.shape
+    out = torch.empty((rows, cols), dtype=torch.float16, device=a.device)
+    row_max = torch.empty(rows, dtype=torch.int32, device=a.device)
+    sums = torch.empty((rows, cols // 16), dtype=torch.float16, device=a.device)
+    _lib.check(_lib.library().strata_rows_to_f16_sums(a.data_ptr(), rows, cols, _lib.dtype_id(a.dtype), out.data_ptr(),
+                                                      row_max.data_ptr(), sums.data_ptr(), _lib.stream()),
+               "rows_to_f16_sums")
+    return out, row_max, sums
 
 
 def _tiled_glu(x: torch.Tensor, indices: torch.Tensor, up, gate, down) -> torch.Tensor:
     """The three products of a prompt's pairs through the tiles (strata_mlx/blocks.py:684-694): the pairs sorted by
     expert on the GPU, gate and up in one launch with the SwiGLU (float32 products, rounded once to the activations'
     type) written in slot order, and down written straight to the pairs. bfloat16 rows go to the float16 MFMA
-    scaled by a power of two each (rows_to_f16). Types the fused kernels do not take, and float32, go through
+    scaled by a power of two each (rows_to_f16). Rows the fused kernels do not take, and float32, go through
     tile_matmul and the reference's steps."""
     tiles, token, where, slot_pair, flat = _route(indices, gate.num_experts)
     xs = x.reshape(-1, x.shape[-1]).contiguous()
@@ -728,12 +750,12 @@ def _tiled_glu(x: torch.Tensor, indices: torch.Tensor, up, gate, down) -> torch.
     same = (gate.kind, gate.output_dims, gate.input_dims, gate.num_experts) == (up.kind, up.output_dims,
                                                                                  up.input_dims, up.num_experts)
     if same and _prompt_fused(gate, x.dtype):
-        x16, x_max = rows_to_f16(xs) if x.dtype == torch.bfloat16 else (xs, None)
+        x16, x_max, x_sum = _tile_rows(xs, gate.kind)
         h = torch.empty((n_slots, gate.output_dims), dtype=x.dtype, device=x.device)
-        _lib.check(lib.strata_prompt_gate_up_swiglu(
+        _lib.check(lib.strata_tiles_gate_up_swiglu(
             _lib.kind_id(gate.kind), gate.blocks.data_ptr(), up.blocks.data_ptr(), gate.num_experts, gate.output_dims,
-            gate.input_dims, x16.data_ptr(), _lib.ptr(x_max), token.data_ptr(), tiles.data_ptr(), tiles.numel(),
-            TOKENS_TILE, h.data_ptr(), _lib.dtype_id(x.dtype), _lib.stream()), f"prompt gate/up {gate.kind}")
+            gate.input_dims, x16.data_ptr(), _lib.ptr(x_max), _lib.ptr(x_sum), token.data_ptr(), tiles.data_ptr(),
+            tiles.numel(), TOKENS_TILE, h.data_ptr(), _lib.dtype_id(x.dtype), _lib.stream()), f"prompt gate/up {gate.kind}")
     else:
         a = xs[token.long()]
 
@@ -742,11 +764,11 @@ def _tiled_glu(x: torch.Tensor, indices: torch.Tensor, up, gate, down) -> torch.
 
         h = (torch.nn.functional.silu(product(gate)) * product(up)).to(x.dtype)
     if _prompt_fused(down, x.dtype):
-        h16, h_max = rows_to_f16(h) if x.dtype == torch.bfloat16 else (h, None)
+        h16, h_max, h_sum = _tile_rows(h, down.kind)
         y = torch.empty((flat.numel(), down.output_dims), dtype=x.dtype, device=x.device)
-        _lib.check(lib.strata_prompt_down(
+        _lib.check(lib.strata_tiles_down(
             _lib.kind_id(down.kind), down.blocks.data_ptr(), down.num_experts, down.output_dims, down.input_dims,
-            h16.data_ptr(), _lib.ptr(h_max), tiles.data_ptr(), tiles.numel(), TOKENS_TILE, slot_pair.data_ptr(),
+            h16.data_ptr(), _lib.ptr(h_max), _lib.ptr(h_sum), tiles.data_ptr(), tiles.numel(), TOKENS_TILE, slot_pair.data_ptr(),
             flat.data_ptr(), flat.numel(), y.data_ptr(), _lib.dtype_id(x.dtype), _lib.stream()), f"prompt down {down.kind}")
     else:
         c = tile_matmul(down.blocks, down.kind, (down.num_experts, down.output_dims, down.input_dims), h, tiles)

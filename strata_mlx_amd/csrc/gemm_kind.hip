@@ -40,25 +40,17 @@ int STRATA_CAT(gemm_launch_, STRATA_KIND)(GemmParams& p, int a_dtype, hipStream_
 namespace strata_prompt {
 
 int STRATA_CAT(prompt_launch_, STRATA_KIND)(PromptParams& p, int mode, int out_dtype, hipStream_t s) {
-  if constexpr (strata_mv::FastTraits<STRATA_KIND>::supported) {
-    if (mode == PM_GLU) {
-      if (out_dtype == DT_F16) return launch_prompt_split<STRATA_KIND, PM_GLU, f16>(p, s);
-      if (out_dtype == DT_BF16) return launch_prompt_split<STRATA_KIND, PM_GLU, bf16_t>(p, s);
-      return STRATA_ERR_DTYPE;
-    }
-    if (mode == PM_SCATTER) {
-      if (out_dtype == DT_F16) return launch_prompt_split<STRATA_KIND, PM_SCATTER, f16>(p, s);
-      if (out_dtype == DT_BF16) return launch_prompt_split<STRATA_KIND, PM_SCATTER, bf16_t>(p, s);
-      return STRATA_ERR_DTYPE;
-    }
-    return STRATA_ERR_ARG;
-  } else {
-    (void)p;
-    (void)mode;
-    (void)out_dtype;
-    (void)s;
-    return STRATA_ERR_KIND;
+  if (mode == PM_GLU) {
+    if (out_dtype == DT_F16) return launch_prompt_split<STRATA_KIND, PM_GLU, f16>(p, s);
+    if (out_dtype == DT_BF16) return launch_prompt_split<STRATA_KIND, PM_GLU, bf16_t>(p, s);
+    return STRATA_ERR_DTYPE;
   }
+  if (mode == PM_SCATTER) {
+    if (out_dtype == DT_F16) return launch_prompt_split<STRATA_KIND, PM_SCATTER, f16>(p, s);
+    if (out_dtype == DT_BF16) return launch_prompt_split<STRATA_KIND, PM_SCATTER, bf16_t>(p, s);
+    return STRATA_ERR_DTYPE;
+  }
+  return STRATA_ERR_ARG;
 }
 
 }  // namespace strata_prompt

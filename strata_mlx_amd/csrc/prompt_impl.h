@@ -1,5 +1,11 @@
 // The prompt kernels: grouped dequant-matmuls over tiles of 16 slots, each tile one expert's, on CDNA4 MFMA, for
-// IQ3_S, IQ3_XXS and Q2_0 rows of whole 256-weight steps and float16 activations (strata_mlx/blocks.py:583-694).
+// every block type and float16 activations (strata_mlx/blocks.py:583-694). Rows of whole 256-weight steps, or of whole
+// 64-weight run pairs in the types with smaller blocks (a last step of one to three run pairs).
+//
+// The types decoded by byte arithmetic (decode_linear4) fold their integer scales in too, so that what is left for
+// the sums is one d a 256-weight block; Q4_K and Q5_K add one MFMA a step for their mins. A layer of 256 Q4_K / Q6_K
+// experts at 384 tokens (1536 x 4096, top-8, bfloat16): 1370 us a launch of gate or up through the decode of float32
+// weights into LDS (gemm_impl.h) -> 764 us for both with the SwiGLU; down 1290 -> 684 us.
 //
 // c[s, :] = W[e(s)] . a[s, :]. A workgroup (4 waves) takes a chunk, up to NT = 3 consecutive tiles of one expert
 // (a run of one expert's tiles is cut into chunks of NT from its first tile; the workgroup at a chunk's first tile
@@ -13,7 +19,7 @@
 // lane each); the K order of an MFMA is therefore a permutation of the step's columns, and the slots' activations
 // are read from LDS in that order. The weights reach the MFMA as exact float16 integers with the run's own scale
 // folded in: IQ3_S's (1 + 2s) * grid (at most 465), IQ3_XXS's (2s + 1) * grid (at most 1922), Q2_0's d * (c - 1)
-// (d times -1, 0, 1 or 2, exact unless |d| > 32752). What is common to a row's step (IQ3_S's d, IQ3_XXS's d / 4)
+// (d times -1, 0, 1 or 2, exact unless |d| > 32752). What is common to a row's step (IQ3_S's d, IQ3_XXS's d / 4, ...)
 // multiplies the step's float32 sums, so nothing is rounded before the sums. Codebook entries come from LDS as
 // float16 magnitudes; their signs are set in registers (no sign table in LDS).
 //
@@ -40,7 +46,21 @@ typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kStep = 256;           // columns a K step: a 256-weight block of every row (four Q2_0 blocks)
+// A block's bytes and the run pairs' (64 weights') of a step, and whether a step may be partial: a row of a type with
+// blocks of 32 or 64 weights may end on any run pair (640 inputs: two steps and a half).
+template <int KIND>
+constexpr int kStepBytes = KindTraits<KIND>::block_bytes * (kStep / KindTraits<KIND>::per_block);
+template <int KIND>
+constexpr bool kMayPart = KindTraits<KIND>::per_block < kStep;
+// The types with a min to each run of 32 weights (w = d sc c - dmin mn): their min term is a product of its own, the
+// runs' mins times the runs' sums of activations, one MFMA a step (the sums in two float16 parts, 8 runs each).
+template <int KIND>
+constexpr bool kHasMin = KIND == K_Q4_K || KIND == K_Q5_K;
+constexpr int kSumCols = 16;       // float16 sums of a step in a row of PromptParams.a_sum: 8 runs high, 8 low
+constexpr float kSumScale = 32.0f;  // a_sum holds the sums over 32 (a run of values below 2^15 stays below 2^15)
 constexpr int kPitch = kStep + 8;    // float16 a slot's step in LDS: 16 slots' 16-byte reads fall on distinct banks
+template <int KIND>
+constexpr int kSlotCols = kPitch + (kHasMin<KIND> ? kSumCols : 0);  // the same with the step's sums of the slot
 constexpr int kXcds = 8;             // workgroup i runs on XCD i % 8
 constexpr int kMinWaves = 3;         // waves a SIMD the kernels are built for (at most 168 VGPRs)
 
@@ -51,6 +71,7 @@ struct PromptParams {
   const f16* a;                 // float16 activations (a_rows x cols)
   const uint32_t* a_row;        // the activation row of each slot, or null (slot s reads row s)
   const uint32_t* a_max;        // scaled rows: each row's largest magnitude (float bits), or null
+  const f16* a_sum;             // the types with mins: each activation row's sums over its runs (kSumCols a step)
   const uint32_t* tile_expert;  // expert of each tile (>= experts: a tile to leave out)
   const uint32_t* slot_pair;    // scatter form: the output row of each slot (0xffffffff: none)
   void* out;                    // C32: float (slots x rows); SwiGLU: h (slots x rows); scatter: y (pairs x rows)
@@ -83,16 +104,32 @@ __device__ __forceinline__ void fold_run(const RunPair<KIND>& f, int h, int g, u
   for (int i = 0; i < N; ++i) w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, w[i]) * m2);
 }
 
-// What multiplies a row's whole step: IQ3_S d, IQ3_XXS d / 4 (strata_mlx/blocks.py:89-116); Q2_0 has none left.
+// What multiplies a row's whole step: d of the types with blocks of 256 weights, IQ3_XXS d / 4
+// (strata_mlx/blocks.py:78-116, 164-175; gguf.py:150-179, 207-218); the others' d is in the weights.
 template <int KIND>
 __device__ __forceinline__ float step_scale(const RunPair<KIND>& f) {
-  if constexpr (KIND == K_IQ3_S) return strata_mv::half_bits(f.d);
+  if constexpr (KIND == K_IQ3_S || KIND == K_Q6_K || KIND == K_Q3_K) return strata_mv::half_bits(f.d);
   if constexpr (KIND == K_IQ3_XXS) return strata_mv::half_bits(f.d) * 0.25f;
+  if constexpr (KIND == K_Q4_K || KIND == K_Q5_K) return strata_mv::half_bits(f.dd & 0xffff);
+  if constexpr (KIND == K_IQ4_XS) return strata_mv::half_bits(f.dh & 0xffff);
   return 1.0f;
 }
 template <int KIND>
 constexpr bool has_step_scale() {
-  return KIND == K_IQ3_S || KIND == K_IQ3_XXS;
+  return KindTraits<KIND>::per_block == kStep;
+}
+
+// The mins' side of a step's min product, lane (n, g): run 0 .. 7's 6-bit mins of row n as float16 for g = 0 (the sums'
+// high parts) and g = 1 (their low parts), zeros for g = 2, 3 (strata_mlx/gguf.py:174-179).
+template <int KIND>
+__device__ __forceinline__ f16x8 min_operand(const RunPair<KIND>& f, int g) {
+  const uint32_t lo = f.sm[1] & 0x3F3F3F3Fu;
+  const uint32_t hi = ((f.sm[2] >> 4) & 0x0F0F0F0Fu) | ((f.sm[1] >> 2) & 0x30303030u);
+  uint32_t w[4];
+  strata_mv::bytes_to_h2<0>(lo, w);
+  strata_mv::bytes_to_h2<0>(hi, w + 2);
+  const uint32_t keep = g < 2 ? ~0u : 0u;
+  return __builtin_bit_cast(f16x8, u32x4{w[0] & keep, w[1] & keep, w[2] & keep, w[3] & keep});
 }
 
 // The signs of 8 weights (bits of s8, weight j at bit j) put on 8 float16 magnitudes (two codebook entries, whose sign
@@ -111,14 +148,109 @@ __device__ __forceinline__ void put_signs(uint32_t s8, const u32x2& g0, const u3
   w[3] = (m3 & 0x80008000u) | g1[1];
 }
 
+// The linear types' codes become float16 with no table: 0x3C00 | code << 4 is 1 + code / 64 (code < 64), and one
+// packed fma by 64 sc less (64 + bias) sc gives sc (code - bias), rounded once: an exact integer for Q4_K and Q5_K
+// (sc code at most 1953) and Q3_K (at most 128), and for Q6_K where it is below 2048 in magnitude. Eight codes from
+// the high nibbles of two words (c0, c1: code bits 0-3) and the bytes h0, h1 (0x3C and the code's bits 4-5).
+__device__ __forceinline__ void codes_folded(uint32_t c0, uint32_t c1, uint32_t h0, uint32_t h1, h2v mul, h2v add,
+                                             uint32_t (&w)[4]) {
+  const uint32_t v[4] = {__builtin_amdgcn_perm(h0, c0, 0x05010400u), __builtin_amdgcn_perm(h0, c0, 0x07030602u),
+                         __builtin_amdgcn_perm(h1, c1, 0x05010400u), __builtin_amdgcn_perm(h1, c1, 0x07030602u)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    w[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2v, v[i]), mul, add));
+}
+__device__ __forceinline__ h2v both(int v) {  // a float16 pair of a small integer
+  const f16 m = (f16)(int16_t)v;
+  return h2v{m, m};
+}
+
+// decode_folded4 of the types without an IQ3 or Q2_0 codebook.
+template <int KIND>
+__device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, int g, int l, uint32_t (&w)[4],
+                                               const DirectTables<KIND>& t) {
+  const uint32_t hi_nibbles = 0xF0F0F0F0u;
+  if constexpr (KIND == K_Q4_K || KIND == K_Q5_K) {
+    const uint32_t q0 = f.qs[l >> 1][2 * (l & 1)], q1 = f.qs[l >> 1][2 * (l & 1) + 1];
+    const uint32_t c0 = (h ? q0 : q0 << 4) & hi_nibbles, c1 = (h ? q1 : q1 << 4) & hi_nibbles;
+    const int sb = 2 * g + h, tb = 8 * (sb & 3);
+    const uint32_t b0 = (f.sm[0] >> tb) & 255, b2 = (f.sm[2] >> tb) & 255;
+    const uint32_t sc = sb >= 4 ? ((b2 & 15) | ((b0 >> 6) << 4)) : (b0 & 63);
+    const h2v m = both((int)(64 * sc));
+    uint32_t h0 = 0x3C3C3C3Cu, h1 = 0x3C3C3C3Cu;
+    if constexpr (KIND == K_Q5_K) {
+      h0 |= (f.qh[l >> 1][2 * (l & 1)] >> sb) & 0x01010101u;
+      h1 |= (f.qh[l >> 1][2 * (l & 1) + 1] >> sb) & 0x01010101u;
+    }
+    codes_folded(c0, c1, h0, h1, m, -m, w);
+  } else if constexpr (KIND == K_Q6_K) {
+    const int r2 = 2 * ((g & 1) + 2 * h);  // the run's bits in the high-bit bytes
+    const uint32_t q0 = f.ql[l >> 1][2 * (l & 1)], q1 = f.ql[l >> 1][2 * (l & 1) + 1];
+    const uint32_t c0 = (h ? q0 : q0 << 4) & hi_nibbles, c1 = (h ? q1 : q1 << 4) & hi_nibbles;
+    const uint32_t h0 = ((f.qh[l >> 1][2 * (l & 1)] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
+    const uint32_t h1 = ((f.qh[l >> 1][2 * (l & 1) + 1] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
+    const int sc = (int8_t)(f.sc[h] >> (8 * (l >> 1)));  // a scale every 16 weights
+    codes_folded(c0, c1, h0, h1, both(64 * sc), both(-96 * sc), w);
+  } else if constexpr (KIND == K_Q3_K) {
+    const int r = 2 * g + h, qsh = 4 * (g & 1) + 2 * h;
+    uint32_t c[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t q = f.qs[l >> 1][2 * (l & 1) + i] >> qsh, m = f.hm[l >> 1][2 * (l & 1) + i] >> r;
+      c[i] = ((q & 0x03030303u) | ((m & 0x01010101u) << 2)) << 4;
+    }
+    const int p = 2 * h + (l >> 1);  // the lane's 6-bit scale
+    const int sc = (int)(((f.lo >> (8 * p + 4 * (g >> 1))) & 15) | (((f.hi >> (8 * p + 2 * g)) & 3) << 4)) - 32;
+    codes_folded(c[0], c[1], 0x3C3C3C3Cu, 0x3C3C3C3Cu, both(64 * sc), both(-68 * sc), w);
+  } else {
+    f16 m;  // what multiplies the run's codes: d of a block of 32, IQ4_XS the run's 6-bit scale
+    if constexpr (KIND == K_Q8_0) {
+      strata_mv::bytes_to_h2<128>(f.q[2 * h + (l >> 1)][2 * (l & 1)] ^ 0x80808080u, w);
+      strata_mv::bytes_to_h2<128>(f.q[2 * h + (l >> 1)][2 * (l & 1) + 1] ^ 0x80808080u, w + 2);
+      m = __builtin_bit_cast(f16, f.d[h]);
+    } else {
+      const int k = 2 * (l & 1);  // byte i's low nibble is weight i, its high nibble weight 16 + i
+      const uint32_t q0 = f.qs[h][k] >> (4 * (l >> 1)), q1 = f.qs[h][k + 1] >> (4 * (l >> 1));
+      const uint32_t c0 = q0 & 0x0F0F0F0Fu, c1 = q1 & 0x0F0F0F0Fu;
+      if constexpr (KIND == K_Q4_0) {
+        strata_mv::bytes_to_h2<8>(c0, w);
+        strata_mv::bytes_to_h2<8>(c1, w + 2);
+      } else if constexpr (KIND == K_Q5_0) {
+        const uint32_t b0 = ((__builtin_amdgcn_ubfe(f.qh[h], 8 * l, 4) * 0x204081u) & 0x01010101u) << 4;
+        const uint32_t b1 = ((__builtin_amdgcn_ubfe(f.qh[h], 8 * l + 4, 4) * 0x204081u) & 0x01010101u) << 4;
+        strata_mv::bytes_to_h2<16>(c0 | b0, w);
+        strata_mv::bytes_to_h2<16>(c1 | b1, w + 2);
+      } else {  // IQ4_NL, IQ4_XS: two codebook values a lookup (pair_codes_run)
+        const char* base = reinterpret_cast<const char*>(t.kv2);
+        const uint32_t two = 2, t0 = c0 | (c0 >> 4), t1 = c1 | (c1 >> 4);
+        w[0] = *reinterpret_cast<const uint32_t*>(base + strata_mv::byte_shl<0>(t0, two));
+        w[1] = *reinterpret_cast<const uint32_t*>(base + strata_mv::byte_shl<2>(t0, two));
+        w[2] = *reinterpret_cast<const uint32_t*>(base + strata_mv::byte_shl<0>(t1, two));
+        w[3] = *reinterpret_cast<const uint32_t*>(base + strata_mv::byte_shl<2>(t1, two));
+      }
+      if constexpr (KIND == K_IQ4_XS) {
+        const int ib = 2 * g + h;
+        const uint32_t ls = ((f.sl >> (8 * g + 4 * h)) & 15) | (((f.dh >> (16 + 2 * ib)) & 3) << 4);
+        m = (f16)(int16_t)((int)ls - 32);
+      } else {
+        m = __builtin_bit_cast(f16, f.d[h]);
+      }
+    }
+    const h2v m2 = h2v{m, m};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, w[i]) * m2);
+  }
+}
+
 // Group pair l (weights 8 l .. 8 l + 7) of run h of the lane's run pair g, IQ3_XXS, IQ3_S or Q2_0: 4 packed
 // float16 pairs, the run's scale and signs folded in (exact). What the four group pairs of a run share is the same
 // expression for each, computed once where they are unrolled together.
 template <int KIND>
 __device__ __forceinline__ void decode_folded4(const RunPair<KIND>& f, int h, int g, int l, uint32_t (&w)[4],
                                                const DirectTables<KIND>& t) {
-  static_assert(KIND == K_IQ3_XXS || KIND == K_IQ3_S || KIND == K_Q2_0, "the staged types");
-  if constexpr (KIND == K_Q2_0) {  // strata_mlx/blocks.py:58-68: code bytes 2 l, 2 l + 1 of the run, four (c - 1) each
+  if constexpr (strata_mv::DirectKind<KIND>::linear) {
+    decode_linear4<KIND>(f, h, g, l, w, t);
+  } else if constexpr (KIND == K_Q2_0) {  // strata_mlx/blocks.py:58-68: code bytes 2 l, 2 l + 1 of the run, four (c - 1) each
     const uint32_t q = f.qs[2 * h + (l >> 1)];
     const u32x2 c0 = t.q2[(q >> (16 * (l & 1))) & 255];
     const u32x2 c1 = t.q2[(q >> (16 * (l & 1) + 8)) & 255];
@@ -145,14 +277,14 @@ __device__ __forceinline__ void decode_folded4(const RunPair<KIND>& f, int h, in
     const u32x2 g1 = strata_mv::lds_entry(t.grid, strata_mv::word_shl<1>(iw, three));
     put_signs((f.sg[h] >> (8 * l)) & 255u, g0, g1, w);
   }
-  fold_run<KIND, 4>(f, h, g, w);
+  if constexpr (!strata_mv::DirectKind<KIND>::linear) fold_run<KIND, 4>(f, h, g, w);
 }
 
 // Run h of the lane's run pair g: 16 packed float16 pairs, the run's scale and signs folded in (exact).
 template <int KIND>
 __device__ __forceinline__ void decode_folded(const RunPair<KIND>& f, int h, int g, uint32_t (&w)[16],
                                               const DirectTables<KIND>& t) {
-  if constexpr (KIND == K_IQ3_XXS || KIND == K_IQ3_S) {
+  if constexpr (KIND != K_Q2_0) {
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
       uint32_t w4[4];
@@ -220,7 +352,9 @@ __device__ __forceinline__ void write_chunk(const PromptParams& p, const f32x4 (
 }
 
 // One chunk of exactly NTC tiles (NTC at compile time: no per-tile branches between the MFMAs).
-template <int KIND, int MODE, typename OT, int WAVES, int NTC>
+// PART: the rows end within a step (kMayPart): in the last one, lanes past the row's run pairs take its last run pair
+// again and the activations past the row are zeros.
+template <int KIND, int MODE, typename OT, int WAVES, int NTC, bool PART>
 __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTables<KIND>& tab,
                                           f16* a_lds, uint32_t e, int t0, int rb, int tid,
                                           int wave) {
@@ -241,8 +375,13 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
   const uint32_t off0 = (uint32_t)min(row0, p.rows - 1) * (uint32_t)p.row_bytes;
   const uint32_t off1 = (uint32_t)min(row1, p.rows - 1) * (uint32_t)p.row_bytes;
   const LaneOffsets<KIND> o = strata_mv::lane_offsets<KIND>(g);
-  const int nsteps = p.cols / kStep;
-  const uint32_t step_bytes = (uint32_t)(p.row_bytes / nsteps);
+  const int nsteps = PART ? (p.cols + kStep - 1) / kStep : p.cols / kStep;
+  constexpr uint32_t step_bytes = kStepBytes<KIND>;
+  constexpr int kP = kSlotCols<KIND>;
+  // in a partial last step, lane group g's run pair is the last one's: this many bytes before its own
+  const int last_pairs = PART ? (p.cols - (nsteps - 1) * kStep) / 64 : 4;
+  const uint32_t back = PART ? (uint32_t)max(0, g - (last_pairs - 1)) * (step_bytes / 4) : 0u;
+  auto fields_at = [&](int k) { return (uint32_t)k * step_bytes - (PART && k == nsteps - 1 ? back : 0u); };
 
   // the thread's pieces of the activations: (tile, slot, piece) -> global row and LDS place
   const f16* arow[kLoads];
@@ -254,15 +393,38 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
     const int slot = (t0 + i) * 16 + m;
     const uint32_t r = p.a_row ? p.a_row[slot] : (uint32_t)slot;
     arow[q] = p.a + (int64_t)r * p.cols + 8 * piece;
-    adst[q] = (i * 16 + m) * kPitch + 8 * piece;
+    adst[q] = (i * 16 + m) * kP + 8 * piece;
   }
   u32x4 av[kLoads];
+  auto load_av = [&](int k) {
 #pragma unroll
-  for (int q = 0; q < kLoads; ++q) av[q] = *reinterpret_cast<const u32x4*>(arow[q]);
+    for (int q = 0; q < kLoads; ++q) {
+      if constexpr (PART) {
+        const bool in = k * kStep + 8 * ((tid + q * kThreadsWg) % (kStep / 8)) < p.cols;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(arow[q] + (in ? k * kStep : 0));
+        av[q] = in ? v : u32x4{0u, 0u, 0u, 0u};
+      } else {
+        av[q] = *reinterpret_cast<const u32x4*>(arow[q] + k * kStep);
+      }
+    }
+  };
+  // the types with mins: threads 0 .. 32 NTC - 1 bring a slot's 8 high or low sums of the step
+  const f16* srow = nullptr;
+  int sdst = 0;
+  u32x4 sv;
+  if constexpr (kHasMin<KIND>) {
+    const int c = min(tid, 32 * NTC - 1), m = c / 2, part = c % 2;
+    const int slot = t0 * 16 + m;
+    const uint32_t r = p.a_row ? p.a_row[slot] : (uint32_t)slot;
+    srow = p.a_sum + (int64_t)r * (nsteps * kSumCols) + 8 * part;
+    sdst = m * kP + kStep + 8 * part;
+    sv = *reinterpret_cast<const u32x4*>(srow);
+  }
+  load_av(0);
 
   RunPair<KIND> f[2][2];  // [step parity][row group]
-  strata_mv::load_fields<KIND>(mat0, off0, o, f[0][0]);
-  strata_mv::load_fields<KIND>(mat1, off1, o, f[0][1]);
+  strata_mv::load_fields<KIND>(mat0, off0 + fields_at(0), o, f[0][0]);
+  strata_mv::load_fields<KIND>(mat1, off1 + fields_at(0), o, f[0][1]);
 
   f32x4 acc[2][NTC];
 #pragma unroll
@@ -274,15 +436,18 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
       const int k = kb + sp;
       if (k < nsteps) {
         // the next step's fields (past the last step, the last again: unconditional loads)
-        const uint32_t nx = (uint32_t)min(k + 1, nsteps - 1) * step_bytes;
+        const uint32_t nx = fields_at(min(k + 1, nsteps - 1));
         strata_mv::load_fields<KIND>(mat0, off0 + nx, o, f[sp ^ 1][0]);
         strata_mv::load_fields<KIND>(mat1, off1 + nx, o, f[sp ^ 1][1]);
         __syncthreads();  // every wave has read the last step's activations (and the tables are written)
 #pragma unroll
         for (int q = 0; q < kLoads; ++q) *reinterpret_cast<u32x4*>(a_lds + adst[q]) = av[q];
+        if constexpr (kHasMin<KIND>) {
+          if (tid < 32 * NTC) *reinterpret_cast<u32x4*>(a_lds + sdst) = sv;
+        }
         if (k + 1 < nsteps) {
-#pragma unroll
-          for (int q = 0; q < kLoads; ++q) av[q] = *reinterpret_cast<const u32x4*>(arow[q] + (k + 1) * kStep);
+          load_av(k + 1);
+          if constexpr (kHasMin<KIND>) sv = *reinterpret_cast<const u32x4*>(srow + (k + 1) * kSumCols);
         }
         __syncthreads();
 
@@ -292,7 +457,7 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
         auto read_a = [&](f16x8 (&a8)[4][NTC], int h, int q) {
 #pragma unroll
           for (int i = 0; i < NTC; ++i)
-            a8[q][i] = *reinterpret_cast<const f16x8*>(a_lds + (i * 16 + n) * kPitch + a_col<KIND>(g, h, q));
+            a8[q][i] = *reinterpret_cast<const f16x8*>(a_lds + (i * 16 + n) * kP + a_col<KIND>(g, h, q));
         };
         auto mfma_group = [&](const f16x8 (&a8)[NTC], const uint32_t* w0, const uint32_t* w1) {
           const f16x8 b0 = __builtin_bit_cast(f16x8, u32x4{w0[0], w0[1], w0[2], w0[3]});
@@ -308,7 +473,7 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           f16x8 a8[4][NTC];
-          if constexpr (NTC >= 3 && (KIND == K_IQ3_S || KIND == K_IQ3_XXS)) {  // a group pair at a time, as staged
+          if constexpr (NTC >= 3 && KIND != K_Q2_0) {  // a group pair at a time, as staged
             read_a(a8, h, 0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -328,6 +493,23 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
             for (int q = 2; q < 4; ++q) read_a(a8, h, q);
 #pragma unroll
             for (int q = 0; q < 4; ++q) mfma_group(a8[q], w0 + 4 * q, w1 + 4 * q);
+          }
+        }
+        if constexpr (kHasMin<KIND>) {
+          const f16x8 b0 = min_operand<KIND>(f[sp][0], g), b1 = min_operand<KIND>(f[sp][1], g);
+          const float m0 = kSumScale * strata_mv::half_bits(f[sp][0].dd >> 16);
+          const float m1 = kSumScale * strata_mv::half_bits(f[sp][1].dd >> 16);
+#pragma unroll
+          for (int i = 0; i < NTC; ++i) {
+            const f16x8 as = *reinterpret_cast<const f16x8*>(a_lds + (i * 16 + n) * kP + kStep + 8 * (g & 1));
+            const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
+            const f32x4 q0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b0, z, 0, 0, 0);
+            const f32x4 q1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b1, z, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              acc[0][i][j] = __builtin_fmaf(-m0, q0[j], acc[0][i][j]);
+              acc[1][i][j] = __builtin_fmaf(-m1, q1[j], acc[1][i][j]);
+            }
           }
         }
         if constexpr (has_step_scale<KIND>()) {
@@ -374,8 +556,6 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
 // registers, spilled) the kernel ran slower.
 template <int KIND>
 constexpr bool kStagedKind = KIND == K_IQ3_S || KIND == K_IQ3_XXS || KIND == K_Q2_0;
-template <int KIND>
-constexpr int kStepBytes = KIND == K_IQ3_S ? 110 : KIND == K_IQ3_XXS ? 98 : 72;  // Q2_0: four 18-byte blocks
 template <int KIND>
 constexpr int kSlotDwords = (kStepBytes<KIND> + 2) / 4;  // dwords a row's step spans: 28, 25, 18
 template <int KIND>
@@ -635,13 +815,14 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
   write_chunk<MODE, OT, NTC>(p, acc, t0, g, row0, row1);
 }
 
-template <int KIND, int MODE, typename OT, int WAVES, int NT, bool STAGED>
+// PART (rows that end within a step) takes the unstaged body.
+template <int KIND, int MODE, typename OT, int WAVES, int NT, bool STAGED, bool PART>
 __global__ __launch_bounds__(64 * WAVES, kMinWaves) void prompt_kernel(PromptParams p) {
   constexpr int kThreadsWg = 64 * WAVES;
-  constexpr bool kStagedHere = STAGED && kStagedKind<KIND>;
+  constexpr bool kStagedHere = STAGED && !PART && kStagedKind<KIND>;
   __shared__ __attribute__((aligned(16))) uint8_t w_lds[kStagedHere ? WAVES * 2 * kGroupBytes<KIND> : 16];
   __shared__ DirectTables<KIND> tab;
-  __shared__ __attribute__((aligned(16))) f16 a_lds[(kStagedHere ? activation_buffers<NT>() : 1) * NT * 16 * kPitch];
+  __shared__ __attribute__((aligned(16))) f16 a_lds[(kStagedHere ? activation_buffers<NT>() : 1) * NT * 16 * kSlotCols<KIND>];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -709,7 +890,7 @@ __global__ __launch_bounds__(64 * WAVES, kMinWaves) void prompt_kernel(PromptPar
       if constexpr (kStagedHere)
         run_chunk_staged<KIND, MODE, OT, WAVES, NT, NTC>(p, tab, a_lds, w_lds, e, t0, rb, tid, wave);
       else
-        run_chunk<KIND, MODE, OT, WAVES, NTC>(p, tab, a_lds, e, t0, rb, tid, wave);
+        run_chunk<KIND, MODE, OT, WAVES, NTC, PART>(p, tab, a_lds, e, t0, rb, tid, wave);
     }
   };
   switch (nt) {
@@ -729,7 +910,14 @@ constexpr int rows_per_wg(int waves) {
   return (MODE == PM_GLU ? 16 : 32) * waves;
 }
 
-// Whether the prompt kernels take a stack: a type they decode, rows of whole 256-weight steps.
+// Whether the tile kernels take a stack: any type here, rows of whole 256-weight steps, or (blocks of 32 or 64
+// weights) of whole 64-weight run pairs.
+inline bool tiles_take(int kind, int64_t cols) {
+  int per = 0, bb = 0;
+  if (strata_kind_info(kind, &per, &bb)) return false;
+  return cols > 0 && cols % (per < kStep ? 64 : kStep) == 0;
+}
+// The same for the entry points of the three expert types.
 inline bool prompt_takes(int kind, int64_t cols) {
   return (kind == K_IQ3_S || kind == K_IQ3_XXS || kind == K_Q2_0) && cols % kStep == 0 && cols > 0;
 }
@@ -746,15 +934,26 @@ int launch_prompt(PromptParams& p, hipStream_t s) {
   const int64_t grid = tiles * p.row_blocks;
   if (grid <= 0) return STRATA_OK;
   if (grid > 0x7fffffff) return STRATA_ERR_SHAPE;
+  auto go = [&](auto staged, auto part) {
+    hipLaunchKernelGGL((prompt_kernel<KIND, MODE, OT, kWaves, kTiles, decltype(staged)::value, decltype(part)::value>),
+                       dim3((unsigned)grid), dim3(64 * kWaves), 0, s, p);
+  };
   // staged rows read whole dwords: the stacks' bases and a row's bytes multiples of 4
-  const bool staged = kStaged && kStagedKind<KIND> && ((uintptr_t)p.blocks[0] & 3) == 0 && ((uintptr_t)p.blocks[1] & 3) == 0 &&
-                      p.row_bytes % 4 == 0 && p.mat_bytes % 4 == 0;
-  if (staged)
-    hipLaunchKernelGGL((prompt_kernel<KIND, MODE, OT, kWaves, kTiles, true>), dim3((unsigned)grid), dim3(64 * kWaves),
-                       0, s, p);
-  else
-    hipLaunchKernelGGL((prompt_kernel<KIND, MODE, OT, kWaves, kTiles, false>), dim3((unsigned)grid), dim3(64 * kWaves),
-                       0, s, p);
+  const bool aligned = ((uintptr_t)p.blocks[0] & 3) == 0 && ((uintptr_t)p.blocks[1] & 3) == 0 &&
+                       p.row_bytes % 4 == 0 && p.mat_bytes % 4 == 0;
+  if (p.cols % kStep != 0) {
+    if constexpr (kMayPart<KIND>) go(std::false_type(), std::true_type());
+    else return STRATA_ERR_SHAPE;
+  } else {
+    if constexpr (kStaged && kStagedKind<KIND>) {
+      if (aligned) {
+        go(std::true_type(), std::false_type());
+        STRATA_CHECK_LAUNCH();
+        return STRATA_OK;
+      }
+    }
+    go(std::false_type(), std::false_type());
+  }
   STRATA_CHECK_LAUNCH();
   return STRATA_OK;
 }

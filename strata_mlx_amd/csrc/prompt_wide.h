@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kWideThreads, kWideWavesSimd) void prompt_wide_kern
 // one-tile chunks, costs it as much as before.
 template <int MODE>
 inline bool wide_takes(const PromptParams& p) {
-  return (MODE == PM_GLU || MODE == PM_SCATTER) && p.n_tiles <= kWideMaxTiles && ((uintptr_t)p.a & 15) == 0 &&
+  return (MODE == PM_GLU || MODE == PM_SCATTER) && p.cols % kStep == 0 && p.n_tiles <= kWideMaxTiles && ((uintptr_t)p.a & 15) == 0 &&
          p.n_tiles >= 8 * p.experts;
 }
 
