@@ -30,7 +30,13 @@ DENSE = {"Q4_0": (32, 18), "Q5_0": (32, 22), "Q8_0": (32, 34), "Q4_K": (256, 144
 NO_GRID = ("IQ2_S", "IQ2_XS", "IQ2_XXS", "IQ1_M")
 
 TOKENS_TILE = 16  # slots of a tile (strata_mlx/blocks.py:581)
-TILES_FROM = 1600  # (token, expert) pairs from which a prompt goes through tiles (strata_mlx/blocks.py:580)
+# (token, expert) pairs from which float16 activations go through tiles (the reference: 1600, strata_mlx/blocks.py:580).
+# Below, each pair decodes its expert's rows again, above, an expert's rows are decoded once for 16 pairs: 8 tokens
+# of top-8 of 256 experts 130 us a pair at a time against 151 in tiles, 12 tokens 234 against 197, 48 tokens 1241
+# against 374 (IQ3_S, 1536 x 4096); Q4_K / Q6_K 267 against 235, 395 against 314, 2464 against 584.
+TILES_FROM = 65
+TILES_FROM_BF16 = 16  # bfloat16, whose matvec is the generic one: 2 tokens 160 against 97 us, 48 tokens 2021 against 394
+TILES_FROM_ANY = 1600  # what the fused tile kernels do not take (float32, ragged rows)
 MATVEC_GLU_UPTO = 1 << 16  # pairs for which down takes silu(gate) * up itself (the reference: 30)
 
 
@@ -570,6 +576,16 @@ def _lookup_glu(x: torch.Tensor, indices: torch.Tensor, up, gate, down) -> torch
     return out.reshape(*indices.shape, down.output_dims)
 
 
+def _tiles_from(dtype: torch.dtype, up, gate, down) -> int:
+    """Pairs from which `switch_glu` takes the tiles for stacks and activations like these."""
+    same = (gate.kind, gate.output_dims, gate.input_dims, gate.num_experts) == (up.kind, up.output_dims,
+                                                                                 up.input_dims, up.num_experts)
+    table = LOOKUP_GLU and all(lookable(lin, dtype) for lin in (up, gate, down))
+    if table or not (same and _prompt_fused(gate, dtype) and _prompt_fused(down, dtype)):
+        return max(TILES_FROM, TILES_FROM_ANY)
+    return TILES_FROM_BF16 if dtype == torch.bfloat16 else TILES_FROM
+
+
 def switch_glu(x: torch.Tensor, indices: torch.Tensor, up: BlockSwitchLinear, gate: BlockSwitchLinear,
                down: BlockSwitchLinear) -> torch.Tensor:
     """down(silu(gate(x)) * up(x)) through each token's experts: x (..., in), indices (..., k) -> (..., k, out).
@@ -577,15 +593,15 @@ def switch_glu(x: torch.Tensor, indices: torch.Tensor, up: BlockSwitchLinear, ga
 
     Decode windows take the matvec kernels: gate and up in one launch reading x once and writing silu(gate) * up
     (rounded as mlx-lm rounds it), then down on that; Q2_0 stacks over float16 too, unless LOOKUP_GLU sends them to
-    the table of sums as the reference's dispatch does (blocks.py:963-964). Prompt chunks (from TILES_FROM pairs) take
+    the table of sums as the reference's dispatch does (blocks.py:963-964). Batches and prompts (from _tiles_from pairs) take
     the tiles: the pairs sorted by expert on the GPU, gate and up with the SwiGLU in one MFMA launch, down written
     straight to the pairs."""
     indices = torch.as_tensor(indices, device=x.device)
     k = indices.shape[-1] if indices.ndim else 1
     flat = indices.reshape(-1)
     xs = x.reshape(-1, x.shape[-1])
-    if flat.numel() >= TILES_FROM and all(tileable(lin.kind, lin.output_dims, lin.input_dims)
-                                          for lin in (up, gate, down)):
+    if flat.numel() >= min(TILES_FROM, TILES_FROM_BF16) and flat.numel() >= _tiles_from(x.dtype, up, gate, down) and \
+            all(tileable(lin.kind, lin.output_dims, lin.input_dims) for lin in (up, gate, down)):
         return _tiled_glu(x, indices, up, gate, down)
     if LOOKUP_GLU and flat.numel() >= LOOKUP_FROM and all(lookable(lin, x.dtype) for lin in (up, gate, down)):
         return _lookup_glu(x, indices, up, gate, down)

@@ -146,14 +146,6 @@ __global__ __launch_bounds__(256) void rows_from_f32_kernel(const float* c, int 
   }
 }
 
-// Rows of y for the pairs naming no expert: NaN, as every matvec gives them.
-template <typename OT>
-__global__ __launch_bounds__(256) void nan_rows_kernel(const uint32_t* idx, int64_t experts, int cols, OT* y) {
-  const int64_t p = blockIdx.x;
-  if (idx[p] < (uint64_t)experts) return;
-  for (int c = threadIdx.x; c < cols; c += 256) y[p * cols + c] = from_f32<OT>(__builtin_nanf(""));
-}
-
 int dispatch(int kind, PromptParams& p, int mode, int out_dtype, hipStream_t s) {
   switch (kind) {
 #define STRATA_CASE(K) \
@@ -321,14 +313,6 @@ static int scatter_down(bool taken, int kind, const void* blocks, int64_t expert
   if (pairs == 0 || rows == 0) return STRATA_OK;
   if (!blocks || !idx || !y || (n_tiles > 0 && (!h || !tile_expert || !slot_pair || (has_min(kind) && !h_sum))))
     return STRATA_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  if (y_dtype == DT_F16)
-    hipLaunchKernelGGL((nan_rows_kernel<f16>), dim3((unsigned)pairs), dim3(256), 0, s, idx, experts, (int)rows, (f16*)y);
-  else
-    hipLaunchKernelGGL((nan_rows_kernel<bf16_t>), dim3((unsigned)pairs), dim3(256), 0, s, idx, experts, (int)rows,
-                       (bf16_t*)y);
-  STRATA_CHECK_LAUNCH();
-  if (n_tiles == 0) return STRATA_OK;
   PromptParams p = {};
   fill_shape(p, kind, experts, rows, cols, n_tiles);
   p.blocks[0] = (const uint8_t*)blocks;
@@ -337,8 +321,10 @@ static int scatter_down(bool taken, int kind, const void* blocks, int64_t expert
   p.a_sum = (const f16*)h_sum;
   p.tile_expert = tile_expert;
   p.slot_pair = slot_pair;
+  p.idx = idx;
+  p.pairs = (int)pairs;
   p.out = y;
-  return dispatch(kind, p, PM_SCATTER, y_dtype, s);
+  return dispatch(kind, p, PM_SCATTER, y_dtype, (hipStream_t)stream);
 }
 
 extern "C" int strata_prompt_gate_up_swiglu(int kind, const void* gate, const void* up, int64_t experts, int64_t rows,

@@ -74,6 +74,8 @@ struct PromptParams {
   const f16* a_sum;             // the types with mins: each activation row's sums over its runs (kSumCols a step)
   const uint32_t* tile_expert;  // expert of each tile (>= experts: a tile to leave out)
   const uint32_t* slot_pair;    // scatter form: the output row of each slot (0xffffffff: none)
+  const uint32_t* idx;          // scatter form: the pairs' experts (a pair naming none gets a row of NaN)
+  int pairs;
   void* out;                    // C32: float (slots x rows); SwiGLU: h (slots x rows); scatter: y (pairs x rows)
   int64_t experts, mat_bytes;
   int rows, cols, row_bytes, n_tiles, row_blocks;
@@ -830,11 +832,18 @@ __global__ __launch_bounds__(64 * WAVES, kMinWaves) void prompt_kernel(PromptPar
   // (tile, row block) of this workgroup: windows of NT tiles dealt to the XCDs in turn (every row block of a
   // window's tiles on one XCD), so that the chunks, which start at the windows, spread evenly
   const int L = blockIdx.x, xcd = L % kXcds, s = L / kXcds;
-  const int per_window = NT * p.row_blocks;
+  const int per_window = NT * p.row_blocks;  // (at least one row block: rows > 0)
   const int w = kXcds * (s / per_window) + xcd, j = (s / p.row_blocks) % NT, rb = s % p.row_blocks;
   const int t0 = w * NT + j;
+  const uint32_t e = t0 < p.n_tiles ? p.tile_expert[t0] : 0xffffffffu;
+  if constexpr (MODE == PM_SCATTER) {  // the pairs naming no expert, one a workgroup (there are more workgroups)
+    for (int q = L; q < p.pairs; q += gridDim.x) {
+      if (p.idx[q] < (uint64_t)p.experts) continue;
+      OT* y = reinterpret_cast<OT*>(p.out) + (int64_t)q * p.rows;
+      for (int c = tid; c < p.rows; c += kThreadsWg) y[c] = from_f32<OT>(__builtin_nanf(""));
+    }
+  }
   if (t0 >= p.n_tiles) return;
-  const uint32_t e = p.tile_expert[t0];
   if (e >= (uint64_t)p.experts) return;  // a tile nothing fills: left out
   // A run of one expert's consecutive tiles is cut into chunks of NT from its first tile: this workgroup works if
   // the run's tiles before t0 are a multiple of NT. The first round looks at the 64 tiles before t0 (lane l at
@@ -931,7 +940,8 @@ int launch_prompt(PromptParams& p, hipStream_t s) {
   constexpr int rpw = rows_per_wg<MODE>(kWaves);
   p.row_blocks = (p.rows + rpw - 1) / rpw;
   const int64_t tiles = (p.n_tiles + kXcds * kTiles - 1) / (kXcds * kTiles) * (kXcds * kTiles);
-  const int64_t grid = tiles * p.row_blocks;
+  int64_t grid = tiles * p.row_blocks;
+  if (MODE == PM_SCATTER && grid == 0) grid = p.pairs;  // no tiles: the rows of pairs naming no expert
   if (grid <= 0) return STRATA_OK;
   if (grid > 0x7fffffff) return STRATA_ERR_SHAPE;
   auto go = [&](auto staged, auto part) {

@@ -9,7 +9,8 @@
 //          prefix over experts (the expert's first tile), tile_expert, and every slot made empty
 //   place  each pair's rank among its block's pairs of the same expert (wave ballots, then the waves
 //          before it), plus its block's offset: the slot; where, token and slot_pair written
-// The tile count is pairs / tile + min(experts, pairs) whatever the routing, as the reference's.
+// The tile count is pairs / tile + min(experts, pairs) whatever the routing, as the reference's. Up to kSmallPairs
+// pairs and kSmallExperts experts, one workgroup does all three in one launch (route_small).
 #include <atomic>
 
 #include "common.h"
@@ -131,6 +132,102 @@ __global__ __launch_bounds__(kBlock) void route_place(const uint32_t* idx, int p
   }
 }
 
+// The three steps by one workgroup: wave w counts and ranks its own run of consecutive pairs, 64 at a time (the lanes
+// naming one expert found bit by bit of the expert's number, a ballot each), with a count per wave and expert in LDS;
+// then per expert the waves' exclusive prefix and the tiles; then each pair's slot. Every slot is written once: an
+// expert's empty slots and the unused tiles' by themselves, no pass that clears them all first. Bound by latency, not
+// by work: three launches take 16-20 us at these sizes (their gaps included), this one 6-9 us (384 to 4096 pairs).
+constexpr int kSmallPairs = 4096, kSmallExperts = 1024, kSmallWaves = 16;
+constexpr int kSmallChunks = kSmallPairs / (64 * kSmallWaves);  // chunks of 64 pairs a wave at most
+
+__global__ __launch_bounds__(64 * kSmallWaves) void route_small(const uint32_t* idx, int pairs, int k, int experts,
+                                                               int tile, int n_tiles, uint32_t* tile_expert,
+                                                               uint32_t* token, uint32_t* where,
+                                                               uint32_t* slot_pair) {
+  extern __shared__ uint32_t sh[];  // [experts] first tiles, then [kSmallWaves][experts] 16-bit counts
+  __shared__ uint32_t wsum[kSmallWaves];
+  uint16_t* cnt = reinterpret_cast<uint16_t*>(sh + experts);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < (kSmallWaves * experts + 1) / 2; i += 64 * kSmallWaves) sh[experts + i] = 0;
+  const int chunks = (pairs + 64 * kSmallWaves - 1) / (64 * kSmallWaves);  // a wave's
+  const int p0 = wave * 64 * chunks + lane;
+  uint32_t ex[kSmallChunks], rank[kSmallChunks];
+#pragma unroll
+  for (int c = 0; c < kSmallChunks; ++c) ex[c] = c < chunks && p0 + 64 * c < pairs ? idx[p0 + 64 * c] : kNone;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < kSmallChunks; ++c) {
+    if (c >= chunks) break;
+    const uint32_t e = ex[c];
+    const bool valid = e < (uint32_t)experts;
+    uint64_t mine = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 10; ++b) {
+      const uint64_t m = __ballot((e >> b) & 1);
+      mine &= (e >> b) & 1 ? m : ~m;
+    }
+    const uint64_t below = mine & ((1ull << lane) - 1);
+    uint32_t base = 0;
+    if (valid) base = cnt[wave * experts + e];  // the wave's pairs of e in its chunks before this one
+    __builtin_amdgcn_wave_barrier();  // every lane has read before the first of them adds the chunk's
+    if (valid && below == 0) cnt[wave * experts + e] = (uint16_t)(base + __popcll(mine));
+    __builtin_amdgcn_wave_barrier();
+    rank[c] = base + (uint32_t)__popcll(below);
+  }
+  __syncthreads();
+  // per expert (experts <= threads): the waves' exclusive prefix, then its tiles and their prefix over the experts
+  uint32_t total = 0;
+  if (tid < experts) {
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) {
+      const uint32_t n = cnt[w * experts + tid];
+      cnt[w * experts + tid] = (uint16_t)total;
+      total += n;
+    }
+  }
+  const uint32_t own = (total + tile - 1) / tile;
+  uint32_t v = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)v, d);
+    if (lane >= d) v += t;
+  }
+  if (lane == 63) wsum[wave] = v;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+  for (int w = 0; w < kSmallWaves; ++w) {
+    before += w < wave ? wsum[w] : 0u;
+    all += wsum[w];
+  }
+  const uint32_t first = before + v - own;
+  auto empty = [&](uint32_t s) {
+    token[s] = 0;
+    if (slot_pair) slot_pair[s] = kNone;
+  };
+  if (tid < experts) {
+    sh[tid] = first;
+    for (uint32_t t = first; t < first + own; ++t) tile_expert[t] = (uint32_t)tid;
+    for (uint32_t s = first * tile + total; s < (first + own) * tile; ++s) empty(s);
+  }
+  for (uint32_t t = all + tid; t < (uint32_t)n_tiles; t += 64 * kSmallWaves) tile_expert[t] = (uint32_t)experts;
+  for (uint32_t s = all * tile + tid; s < (uint32_t)n_tiles * tile; s += 64 * kSmallWaves) empty(s);
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < kSmallChunks; ++c) {
+    const int p = p0 + 64 * c;
+    if (c >= chunks || p >= pairs) break;
+    const uint32_t e = ex[c];
+    if (e >= (uint32_t)experts) {
+      where[p] = kNone;
+      continue;
+    }
+    const uint32_t slot = sh[e] * tile + cnt[wave * experts + e] + rank[c];
+    where[p] = slot;
+    token[slot] = (uint32_t)(p / k);
+    if (slot_pair) slot_pair[slot] = (uint32_t)p;
+  }
+}
+
 // The workspace of strata_route_tiles_noalloc: the library's own device memory, sized for its largest call. Every
 // word the kernels read is written by the same call first (the counts by route_count, the first tiles by
 // route_scan), so the array needs no clearing between calls; calls that overlap on one GPU share it and race.
@@ -179,6 +276,13 @@ int strata_route_tiles(const uint32_t* idx, int64_t pairs, int64_t k, int64_t ex
   if (n_tiles == 0) return STRATA_OK;
   if (!tile_expert || !token || !workspace || (pairs > 0 && (!idx || !where))) return STRATA_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
+  if (pairs <= kSmallPairs && experts <= kSmallExperts) {
+    const size_t lds = (size_t)experts * sizeof(uint32_t) + (kSmallWaves * (size_t)experts + 1) / 2 * sizeof(uint32_t);
+    hipLaunchKernelGGL(route_small, dim3(1), dim3(64 * kSmallWaves), lds, s, idx, (int)pairs, (int)k, (int)experts,
+                       (int)tile, (int)n_tiles, tile_expert, token, where, slot_pair);
+    STRATA_CHECK_LAUNCH();
+    return STRATA_OK;
+  }
   const int nblocks = (int)((pairs + kBlock - 1) / kBlock);
   uint32_t* blk = (uint32_t*)workspace;
   uint32_t* first_tile = blk + (int64_t)nblocks * experts;

@@ -94,3 +94,27 @@ def test_a_token_far_from_float16s_range(gpu):
     want = torch.stack([w[i % 2] @ h[i].double() for i in range(40)])
     err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
     assert float(err.max()) <= 2.0**-8
+
+
+@pytest.mark.parametrize("pairs, experts", [(1, 1), (63, 5), (64, 256), (65, 1024), (1023, 7), (1025, 512), (2500, 3),
+                                            (4096, 256), (4097, 256), (4000, 1025)])
+def test_routes_of_one_workgroup_and_of_three_launches(gpu, pairs, experts):
+    """tiles_of's layout with every slot's pair, at the sizes around the one-launch form's limits (4096 pairs, 1024
+    experts) and a wave's chunks of 64, some pairs naming no expert."""
+    rng = np.random.default_rng(pairs + experts)
+    idx = rng.integers(0, experts, (pairs, 1))
+    idx[rng.random(pairs) < 0.03] = experts + 3
+    tiles, token, where, slot_pair, _ = (t.cpu().numpy() for t in B._route(torch.from_numpy(idx).to(gpu), experts))
+    flat, tile = idx[:, 0], B.TOKENS_TILE
+    counts = np.bincount(flat[flat < experts], minlength=experts)
+    per = (counts + tile - 1) // tile
+    first = np.concatenate([[0], np.cumsum(per)])
+    assert np.array_equal(tiles, np.concatenate([np.repeat(np.arange(experts), per),
+                                                 np.full(len(tiles) - first[-1], experts)]))
+    slots = np.full(len(tiles) * tile, -1)
+    for e in np.unique(flat[flat < experts]):
+        at = np.nonzero(flat == e)[0]
+        slots[first[e] * tile:first[e] * tile + len(at)] = at
+        assert np.array_equal(where[at], first[e] * tile + np.arange(len(at)))
+    assert np.array_equal(slot_pair, slots) and (where[flat >= experts] == -1).all()
+    assert np.array_equal(token, np.where(slots >= 0, slots, 0))
