@@ -40,6 +40,10 @@ TILES_FROM_ANY = 1600  # what the fused tile kernels do not take (float32, ragge
 MATVEC_GLU_UPTO = 1 << 16  # pairs for which down takes silu(gate) * up itself (the reference: 30)
 
 
+def block_weights(kind: str) -> int:
+    return {**BLOCK, **DENSE}[kind][0]
+
+
 def row_bytes(kind: str, cols: int) -> int:
     per_block, block_bytes = {**BLOCK, **DENSE}[kind]
     if cols % per_block:
@@ -730,9 +734,8 @@ MIN_KINDS = ("Q4_K", "Q5_K")  # types with a min to each run, whose tile kernels
 def _prompt_fused(lin, dtype: torch.dtype) -> bool:
     """Stacks the fused tile kernels take: 16-bit activations, rows of whole 256-weight steps, or of whole 64-weight
     run pairs in the types with smaller blocks; a matrix below 4 GiB (32-bit row offsets)."""
-    per_block = {**BLOCK, **DENSE}[lin.kind][0]
     return (dtype in (torch.float16, torch.bfloat16) and lin.kind not in NO_GRID
-            and lin.input_dims % (64 if per_block < 256 else 256) == 0
+            and lin.input_dims % (64 if block_weights(lin.kind) < 256 else 256) == 0
             and lin.output_dims * lin.row_bytes < 1 << 32)
 
 

@@ -2,6 +2,7 @@
 #include "gemm_impl.h"
 #include "prompt_impl.h"
 #include "prompt_wide.h"
+#include "window_impl.h"
 
 #ifndef STRATA_KIND
 #error "STRATA_KIND must name a GGUF type id"
@@ -54,3 +55,11 @@ int STRATA_CAT(prompt_launch_, STRATA_KIND)(PromptParams& p, int mode, int out_d
 }
 
 }  // namespace strata_prompt
+
+namespace strata_window {
+
+int STRATA_CAT(window_launch_, STRATA_KIND)(const WindowParams& p, int dtype, hipStream_t s) {
+  return dtype == DT_F16 ? launch_window<STRATA_KIND, f16>(p, s) : launch_window<STRATA_KIND, bf16_t>(p, s);
+}
+
+}  // namespace strata_window

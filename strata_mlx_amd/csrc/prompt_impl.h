@@ -167,10 +167,28 @@ __device__ __forceinline__ h2v both(int v) {  // a float16 pair of a small integ
   return h2v{m, m};
 }
 
-// decode_folded4 of the types without an IQ3 or Q2_0 codebook.
+// The types whose folded weights may need more than float16's 11 bits: Q6_K (sc (code - 32) up to 4096), IQ4_XS (up to
+// 4064), and those with a float16 d in the weights.
 template <int KIND>
+constexpr bool kInexact = KIND == K_Q6_K || KIND == K_IQ4_XS || KIND == K_Q8_0 || KIND == K_IQ4_NL || KIND == K_Q4_0 ||
+                          KIND == K_Q5_0;
+
+// The products e m of four packed pairs of integers: rounded once into w; SPLIT: and what the rounding left into lo.
+template <bool SPLIT>
+__device__ __forceinline__ void fold_pairs(uint32_t (&w)[4], h2v m, uint32_t (&lo)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const h2v e = __builtin_bit_cast(h2v, w[i]), v = e * m;
+    w[i] = __builtin_bit_cast(uint32_t, v);
+    if constexpr (SPLIT) lo[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, m, -v));
+  }
+}
+
+// decode_folded4 of the types without an IQ3 or Q2_0 codebook; SPLIT (kInexact): the weights as w + lo.
+template <int KIND, bool SPLIT = false>
 __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, int g, int l, uint32_t (&w)[4],
-                                               const DirectTables<KIND>& t) {
+                                               uint32_t (&lo)[4], const DirectTables<KIND>& t) {
+  static_assert(!SPLIT || kInexact<KIND>, "the other types' weights are exact");
   const uint32_t hi_nibbles = 0xF0F0F0F0u;
   if constexpr (KIND == K_Q4_K || KIND == K_Q5_K) {
     const uint32_t q0 = f.qs[l >> 1][2 * (l & 1)], q1 = f.qs[l >> 1][2 * (l & 1) + 1];
@@ -192,7 +210,12 @@ __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, in
     const uint32_t h0 = ((f.qh[l >> 1][2 * (l & 1)] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
     const uint32_t h1 = ((f.qh[l >> 1][2 * (l & 1) + 1] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
     const int sc = (int8_t)(f.sc[h] >> (8 * (l >> 1)));  // a scale every 16 weights
-    codes_folded(c0, c1, h0, h1, both(64 * sc), both(-96 * sc), w);
+    if constexpr (SPLIT) {  // the integers code - 32, then their products
+      codes_folded(c0, c1, h0, h1, both(64), both(-96), w);
+      fold_pairs<true>(w, both(sc), lo);
+    } else {
+      codes_folded(c0, c1, h0, h1, both(64 * sc), both(-96 * sc), w);
+    }
   } else if constexpr (KIND == K_Q3_K) {
     const int r = 2 * g + h, qsh = 4 * (g & 1) + 2 * h;
     uint32_t c[2];
@@ -238,9 +261,7 @@ __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, in
         m = __builtin_bit_cast(f16, f.d[h]);
       }
     }
-    const h2v m2 = h2v{m, m};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, w[i]) * m2);
+    fold_pairs<SPLIT>(w, h2v{m, m}, lo);
   }
 }
 
@@ -251,7 +272,8 @@ template <int KIND>
 __device__ __forceinline__ void decode_folded4(const RunPair<KIND>& f, int h, int g, int l, uint32_t (&w)[4],
                                                const DirectTables<KIND>& t) {
   if constexpr (strata_mv::DirectKind<KIND>::linear) {
-    decode_linear4<KIND>(f, h, g, l, w, t);
+    uint32_t lo[4];
+    decode_linear4<KIND>(f, h, g, l, w, lo, t);
   } else if constexpr (KIND == K_Q2_0) {  // strata_mlx/blocks.py:58-68: code bytes 2 l, 2 l + 1 of the run, four (c - 1) each
     const uint32_t q = f.qs[2 * h + (l >> 1)];
     const u32x2 c0 = t.q2[(q >> (16 * (l & 1))) & 255];

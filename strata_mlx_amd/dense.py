@@ -8,7 +8,7 @@
                    (blocks.q3k_planes), as the reference holds them.
     BlockEmbedding rows of an embedding decoded when their tokens come (dense.py:245-258).
 
-Up to MAX_TOKENS tokens a product is a window of the matvec kernel (each block decoded once for every token). A
+Up to MAX_TOKENS tokens (WINDOW_TOKENS in 16 bits) a product is a window, each block decoded once for every token. A
 longer chunk (a prompt's) of float16 or bfloat16 tokens is multiplied as the reference multiplies it
 (dense.py:234-241): the layer dequantized for the chunk (strata_dequantize, each weight exact in float32 and
 rounded once to float16) and let go, then a library product with float32 sums (torch.mm; 4-6 times the tile
@@ -21,6 +21,8 @@ import torch
 from . import blocks as B
 
 MAX_TOKENS = 8  # more than a window: a chunk of a prompt, multiplied as floats (dense.py:33)
+# the same for 16-bit tokens and rows of at most WINDOW_COLS inputs: what the MFMA window kernel takes in one pass
+WINDOW_TOKENS, WINDOW_COLS = 16, 4096
 # Q3_K layers held as planes (blocks.q3k_planes), as the reference holds them (dense.py:190, 214-215), when True;
 # by default they stay the file's blocks, which the register decode reads at twice the planes window's speed
 PLANES = False
@@ -92,7 +94,9 @@ class BlockLinear:
                 out = x2 @ self.floats(x.dtype).T
             if row_ids is not None:
                 out = out[:, row_ids.reshape(-1).long()]
-        elif tokens <= MAX_TOKENS or row_ids is not None:
+        elif tokens <= MAX_TOKENS or row_ids is not None or (
+                tokens <= WINDOW_TOKENS and cols <= WINDOW_COLS and x2.dtype != torch.float32
+                and cols % (64 if B.block_weights(self.kind) < 256 else 256) == 0):
             out = B.window_matvec(self.blocks, self.kind, rows, cols, x2, row_ids=row_ids)
         elif x2.dtype in (torch.float16, torch.bfloat16):
             out = float16_chunk(self.floats(torch.float16), x2)
