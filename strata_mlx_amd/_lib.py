@@ -53,6 +53,8 @@ SIGNATURES = {
     "strata_expert_matvec_swiglu": (_i, [_i, _p, _i64, _i64, _i64, _p, _i64, _p, _p, _i, _p, _p]),
     "strata_expert_matvec_ptrs": (_i, [_i, _p, _i64, _i64, _i64, _p, _i, _i64, _p, _p]),
     "strata_dense_matvec": (_i, [_i, _p, _i64, _i64, _p, _i64, _i, _p, _i, _p, _i64, _p]),
+    "strata_dense_chunk_workspace": (_i64, [_i64, _i64]),
+    "strata_dense_chunk": (_i, [_i, _p, _i64, _i64, _p, _i64, _i, _p, _p, _p]),
     "strata_route_tiles_max": (_i64, [_i64, _i64, _i64]),
     "strata_route_tiles_workspace": (_i64, [_i64, _i64]),
     "strata_route_tiles": (_i, [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]),

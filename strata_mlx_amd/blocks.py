@@ -386,6 +386,23 @@ def window_matvec(blocks: torch.Tensor, kind: str, rows: int, cols: int, x: torc
     return out
 
 
+def chunk_matmul(blocks: torch.Tensor, kind: str, rows: int, cols: int, x: torch.Tensor) -> torch.Tensor:
+    """out[t] = W . x[t] for one layer `blocks` of (rows, cols) and a chunk x (tokens, cols) of float16 or bfloat16
+    tokens, on MFMA straight from the blocks (weights rounded to float16, float32 sums): (tokens, rows) in x's type.
+    The product of strata_mlx/dense.py:234-242 without the unpacked weights."""
+    _flat_u8(blocks)
+    x2 = x.reshape(-1, cols).contiguous()
+    if x2.data_ptr() % 16:
+        x2 = x2.clone()
+    tokens, lib = x2.shape[0], _lib.library()
+    out = torch.empty((tokens, rows), dtype=x.dtype, device=x.device)
+    ws = torch.empty(lib.strata_dense_chunk_workspace(tokens, cols), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.strata_dense_chunk(_lib.kind_id(kind), blocks.data_ptr(), rows, cols, x2.data_ptr(), tokens,
+                                      _lib.dtype_id(x.dtype), out.data_ptr(), ws.data_ptr(), _lib.stream()),
+               f"chunk {kind}")
+    return out
+
+
 # ---- Q3_K held as planes (strata_mlx/blocks.py:397-512): the blocks rearranged once into aligned arrays of their
 # parts (high-bit words, value words, decoded scales, d), 114 bytes a block where the file has 110.
 

@@ -1,5 +1,6 @@
 // C-ABI entry point of the prompt kernel (declared in include/strata_gfx950.h); kernels in gemm_impl.h.
 #include "gemm_impl.h"
+#include "chunk_impl.h"
 
 namespace strata_gemm {
 #define STRATA_DECLARE(K) int gemm_launch_##K(GemmParams&, int, hipStream_t);
@@ -58,6 +59,69 @@ extern "C" int strata_grouped_matmul(int kind, const void* blocks, int64_t exper
     STRATA_CASE(20)
     STRATA_CASE(21)
     STRATA_CASE(13)
+    STRATA_CASE(23)
+    STRATA_CASE(42)
+#undef STRATA_CASE
+    default: return STRATA_ERR_KIND;
+  }
+}
+
+namespace strata_chunk {
+#define STRATA_DECLARE(K) int chunk_launch_##K(ChunkParams&, const void*, int, void*, hipStream_t);
+STRATA_DECLARE(2)
+STRATA_DECLARE(6)
+STRATA_DECLARE(8)
+STRATA_DECLARE(11)
+STRATA_DECLARE(12)
+STRATA_DECLARE(13)
+STRATA_DECLARE(14)
+STRATA_DECLARE(18)
+STRATA_DECLARE(20)
+STRATA_DECLARE(21)
+STRATA_DECLARE(23)
+STRATA_DECLARE(42)
+#undef STRATA_DECLARE
+}  // namespace strata_chunk
+
+extern "C" int64_t strata_dense_chunk_workspace(int64_t tokens, int64_t cols) {
+  if (tokens < 0 || cols < 0) return 0;
+  return strata_chunk::chunk_workspace(tokens, cols);
+}
+
+extern "C" int strata_dense_chunk(int kind, const void* blocks, int64_t rows, int64_t cols, const void* x,
+                                  int64_t tokens, int dtype, void* out, void* workspace, void* stream) {
+  int per = 0, bb = 0;
+  if (strata_kind_info(kind, &per, &bb)) return STRATA_ERR_KIND;
+  if (dtype != DT_F16 && dtype != DT_BF16) return STRATA_ERR_DTYPE;
+  if (rows < 0 || tokens < 0) return STRATA_ERR_ARG;
+  // row offsets in the matrix are 32-bit
+  if (!strata_prompt::tiles_take(kind, cols) || rows > (1 << 24) || cols > (1 << 20) || tokens > (1 << 20) ||
+      rows * (cols / per * bb) >= (int64_t(1) << 32))
+    return STRATA_ERR_SHAPE;
+  if (rows == 0 || tokens == 0) return STRATA_OK;
+  if (!blocks || !x || !out || !workspace || ((uintptr_t)x & 15) || ((uintptr_t)workspace & 15)) return STRATA_ERR_ARG;
+  strata_chunk::ChunkParams p = {};
+  p.blocks = (const uint8_t*)blocks;
+  p.out = out;
+  p.rows = (int)rows;
+  p.cols = (int)cols;
+  p.row_bytes = (int)(cols / per * bb);
+  p.tokens = (int)tokens;
+  p.nsteps = (int)((cols + strata_prompt::kStep - 1) / strata_prompt::kStep);
+  hipStream_t s = (hipStream_t)stream;
+  switch (kind) {
+#define STRATA_CASE(K) \
+  case K: return strata_chunk::chunk_launch_##K(p, x, dtype, workspace, s);
+    STRATA_CASE(2)
+    STRATA_CASE(6)
+    STRATA_CASE(8)
+    STRATA_CASE(11)
+    STRATA_CASE(12)
+    STRATA_CASE(13)
+    STRATA_CASE(14)
+    STRATA_CASE(18)
+    STRATA_CASE(20)
+    STRATA_CASE(21)
     STRATA_CASE(23)
     STRATA_CASE(42)
 #undef STRATA_CASE

@@ -3,6 +3,7 @@
 #include "prompt_impl.h"
 #include "prompt_wide.h"
 #include "window_impl.h"
+#include "chunk_impl.h"
 
 #ifndef STRATA_KIND
 #error "STRATA_KIND must name a GGUF type id"
@@ -63,3 +64,12 @@ int STRATA_CAT(window_launch_, STRATA_KIND)(const WindowParams& p, int dtype, hi
 }
 
 }  // namespace strata_window
+
+namespace strata_chunk {
+
+int STRATA_CAT(chunk_launch_, STRATA_KIND)(ChunkParams& p, const void* x, int dtype, void* workspace, hipStream_t s) {
+  return dtype == DT_F16 ? launch_chunk<STRATA_KIND, f16>(p, x, workspace, s)
+                         : launch_chunk<STRATA_KIND, bf16_t>(p, x, workspace, s);
+}
+
+}  // namespace strata_chunk

@@ -62,7 +62,9 @@ constexpr int kPitch = kStep + 8;    // float16 a slot's step in LDS: 16 slots' 
 template <int KIND>
 constexpr int kSlotCols = kPitch + (kHasMin<KIND> ? kSumCols : 0);  // the same with the step's sums of the slot
 constexpr int kXcds = 8;             // workgroup i runs on XCD i % 8
-constexpr int kMinWaves = 3;         // waves a SIMD the kernels are built for (at most 168 VGPRs)
+// waves a SIMD the kernels are built for: three (at most 168 VGPRs); two for the types whose fields would spill
+template <int KIND>
+constexpr int kMinWaves = KIND == K_Q4_K || KIND == K_Q5_K || KIND == K_Q6_K || KIND == K_Q3_K || KIND == K_Q8_0 ? 2 : 3;
 
 enum PromptMode : int { PM_C32 = 0, PM_GLU = 1, PM_SCATTER = 2 };
 
@@ -578,14 +580,21 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
 // would also wait for the next step's rows). The LDS (42-44 KB) and the registers (159-167) leave three workgroups
 // on a CU; at two (a third row buffer, or the IQ3_XXS codebook with its signs folded in, 32 KB) or at four (128
 // registers, spilled) the kernel ran slower.
+//
+// Q6_K, IQ4_NL, Q4_0 and Q8_0 rows too (kDwordRows), whose fields lie at 2 or 4 bytes past a boundary: loaded straight
+// into registers, their 16-byte loads ran several times longer than aligned ones. Their slots are an odd number of
+// dwords apart, so that reads of one dword spread over the banks, and each field is put together from dwords. Down of
+// a layer of 256 Q6_K experts at 384 tokens 684 -> DOWN_Q6K us.
 template <int KIND>
-constexpr bool kStagedKind = KIND == K_IQ3_S || KIND == K_IQ3_XXS || KIND == K_Q2_0;
+constexpr bool kDwordRows = KIND == K_Q6_K || KIND == K_IQ4_NL || KIND == K_Q4_0 || KIND == K_Q8_0;
 template <int KIND>
-constexpr int kSlotDwords = (kStepBytes<KIND> + 2) / 4;  // dwords a row's step spans: 28, 25, 18
+constexpr bool kStagedKind = KIND == K_IQ3_S || KIND == K_IQ3_XXS || KIND == K_Q2_0 || kDwordRows<KIND>;
 template <int KIND>
-constexpr int kSlotPitch = KIND == K_Q2_0 ? 20 : 28;     // dwords a row's slot (112 bytes; Q2_0 80)
+constexpr int kSlotDwords = (kStepBytes<KIND> + 2) / 4;  // dwords a row's step spans: 28, 25, 18; 53, 36, 36, 68
 template <int KIND>
-constexpr int kGroupLoads = 16 * kSlotPitch<KIND> / 64;  // wave instructions a group of 16 rows: 7 (Q2_0 5)
+constexpr int kSlotPitch = kDwordRows<KIND> ? kSlotDwords<KIND> | 1 : KIND == K_Q2_0 ? 20 : 28;  // dwords a row's slot
+template <int KIND>
+constexpr int kGroupLoads = (16 * kSlotPitch<KIND> + 63) / 64;  // wave instructions a group of 16 rows: 7 (Q2_0 5)
 template <int KIND>
 constexpr int kGroupBytes = 256 * kGroupLoads<KIND>;     // a group's buffer
 
@@ -654,6 +663,63 @@ __device__ __forceinline__ void lds_fields(const uint8_t* slot, int g, RunPair<K
   }
 }
 
+// N words at an even byte offset of LDS: N + 1 aligned dwords, shifted
+template <int N>
+__device__ __forceinline__ void words_at(const uint8_t* base, uint32_t off, uint32_t (&w)[N]) {
+  uint32_t d[N + 1];
+#pragma unroll
+  for (int k = 0; k <= N; ++k) d[k] = lds_at<uint32_t>(base, (off & ~3u) + 4u * k);
+#pragma unroll
+  for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_alignbyte(d[k + 1], d[k], off & 3u);
+}
+// run pair g's fields of a step that starts at byte `off` of LDS (Q6_K: even; the others a multiple of 4)
+template <int KIND>
+__device__ __forceinline__ void dword_fields(const uint8_t* lds, uint32_t off, int g, RunPair<KIND>& f) {
+  if constexpr (KIND == K_Q6_K) {
+    const LaneOffsets<K_Q6_K> o = strata_mv::lane_offsets<K_Q6_K>(g);
+    uint32_t ql[8], qh[8];
+    words_at<8>(lds, off + o.qs, ql);
+    words_at<8>(lds, off + o.a, qh);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      f.ql[k / 4][k % 4] = ql[k];
+      f.qh[k / 4][k % 4] = qh[k];
+    }
+    f.sc[0] = lds_at<uint16_t>(lds, off + o.b);
+    f.sc[1] = lds_at<uint16_t>(lds, off + o.b + 4);
+    f.d = lds_at<uint16_t>(lds, off + o.d);
+  } else if constexpr (KIND == K_Q8_0) {  // 68 bytes: d, 32 codes, d, 32 codes
+    uint32_t w[17];
+#pragma unroll
+    for (int k = 0; k < 17; ++k) w[k] = lds_at<uint32_t>(lds, off + 68 * g + 4 * k);
+    f.d[0] = (uint16_t)(w[0] & 0xffffu);
+    f.d[1] = (uint16_t)(w[8] >> 16);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      f.q[k / 4][k % 4] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
+      f.q[2 + k / 4][k % 4] = w[9 + k];
+    }
+  } else {
+    static_assert(KIND == K_IQ4_NL || KIND == K_Q4_0, "the dword types");  // 36 bytes: d, 16 code bytes, twice
+    uint32_t w[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) w[k] = lds_at<uint32_t>(lds, off + 36 * g + 4 * k);
+    f.d[0] = (uint16_t)(w[0] & 0xffffu);
+    f.d[1] = (uint16_t)(w[4] >> 16);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      f.qs[0][k] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
+      f.qs[1][k] = w[5 + k];
+    }
+  }
+}
+// The first byte of a dword type's slot at step k: the step's dword, or (a partial last step) as many dwords before
+// the row's end, so that a slot never reaches past its row.
+template <int KIND>
+__device__ __forceinline__ uint32_t dword_first(int k, int row_bytes) {
+  return min((uint32_t)(k * kStepBytes<KIND>) & ~3u, (uint32_t)(row_bytes - 4 * kSlotDwords<KIND>));
+}
+
 // Activation buffers of the staged form: two (one barrier a step) up to chunks of two tiles; for longer chunks one,
 // which keeps the LDS at three workgroups a CU (a second barrier a step waits for its writes).
 template <int NT>
@@ -661,7 +727,7 @@ constexpr int activation_buffers() {
   return NT <= 2 ? 2 : 1;
 }
 
-template <int KIND, int MODE, typename OT, int WAVES, int NT, int NTC>
+template <int KIND, int MODE, typename OT, int WAVES, int NT, int NTC, bool PART>
 __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const DirectTables<KIND>& tab,
                                                  f16* a_lds, uint8_t* w_lds, uint32_t e, int t0, int rb, int tid,
                                                  int wave) {
@@ -671,7 +737,8 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
   constexpr int kChunks = NTC * 16 * (kStep / 8);
   constexpr int kLoads = kChunks / kThreadsWg;
   static_assert(kChunks % kThreadsWg == 0, "whole pieces a thread");
-  static_assert(kStagedKind<KIND>, "staged rows: IQ3_S, IQ3_XXS, Q2_0");
+  static_assert(kStagedKind<KIND> && (!PART || kDwordRows<KIND>), "staged rows");
+  constexpr bool kDwords = kDwordRows<KIND>;
   constexpr int kSB = kStepBytes<KIND>, kDW = kSlotDwords<KIND>, kGL = kGroupLoads<KIND>, kPitchDw = kSlotPitch<KIND>;
   constexpr int kGB = kGroupBytes<KIND>;
   constexpr int kABuf = NT * 16 * kPitch;  // float16: an activation buffer
@@ -684,28 +751,33 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
   const uint8_t* mat[2] = {p.blocks[0] + (int64_t)e * p.mat_bytes,
                            (kGlu ? p.blocks[1] : p.blocks[0]) + (int64_t)e * p.mat_bytes};
   const int grow[2] = {r0, kGlu ? r0 : r0 + 16};  // first row of each group
-  const int nsteps = p.cols / kStep;
+  const int nsteps = PART ? (p.cols + kStep - 1) / kStep : p.cols / kStep;
+  // a partial last step: lane group g's run pair past the row is the row's last
+  const int last_pairs = PART ? (p.cols - (nsteps - 1) * kStep) / 64 : 4;
 
   // the lane's dword of each staging load: row q of the group, dword d of its slot (the slot's spare dwords: the
   // row's last dword again)
-  uint32_t voff[2][kGL];
+  // (kDwords: one set for both groups, whose rows are whole: the launch checks)
+  uint32_t voff[kDwords ? 1 : 2][kGL];
+  if constexpr (kDwords) mat[1] += (int64_t)(grow[1] - grow[0]) * p.row_bytes;
 #pragma unroll
-  for (int grp = 0; grp < 2; ++grp)
+  for (int grp = 0; grp < (kDwords ? 1 : 2); ++grp)
 #pragma unroll
     for (int i = 0; i < kGL; ++i) {
       const int f = 64 * i + lane;
-      const int q = f / kPitchDw, d = min(f % kPitchDw, kDW - 1);
+      const int q = min(f / kPitchDw, 15), d = min(f % kPitchDw, kDW - 1);
       voff[grp][i] = (uint32_t)min(grow[grp] + q, p.rows - 1) * (uint32_t)p.row_bytes + 4u * (uint32_t)d;
     }
   const uint32_t w_base = (uint32_t)(uintptr_t)w_lds;
   auto stage = [&](int k) {
-    const uint32_t first = (uint32_t)(k * kSB) & ~3u;  // the dword holding the step's first byte
+    // the dword holding the step's first byte
+    const uint32_t first = kDwords ? dword_first<KIND>(k, p.row_bytes) : (uint32_t)(k * kSB) & ~3u;
 #pragma unroll
     for (int grp = 0; grp < 2; ++grp) {
       const uint8_t* base = mat[grp] + first;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(w_base + (uint32_t)((wave * 2 + grp) * kGB));
 #pragma unroll
-      for (int i = 0; i < kGL; ++i) dma_dword(base, voff[grp][i], dst + 256u * i);
+      for (int i = 0; i < kGL; ++i) dma_dword(base, voff[kDwords ? 0 : grp][i], dst + 256u * i);
     }
   };
 
@@ -721,17 +793,25 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
     adst[q] = (i * 16 + m) * kPitch + 8 * piece;
   }
   u32x4 av[kLoads];
+  auto load_av = [&](int k) {
 #pragma unroll
-  for (int q = 0; q < kLoads; ++q) av[q] = *reinterpret_cast<const u32x4*>(arow[q]);
+    for (int q = 0; q < kLoads; ++q) {
+      if constexpr (PART) {
+        const bool in = k * kStep + 8 * ((tid + q * kThreadsWg) % (kStep / 8)) < p.cols;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(arow[q] + (in ? k * kStep : 0));
+        av[q] = in ? v : u32x4{0u, 0u, 0u, 0u};
+      } else {
+        av[q] = *reinterpret_cast<const u32x4*>(arow[q] + k * kStep);
+      }
+    }
+  };
+  load_av(0);
   if constexpr (kABufs == 2) {
 #pragma unroll
     for (int q = 0; q < kLoads; ++q) *reinterpret_cast<u32x4*>(a_lds + adst[q]) = av[q];
   }
   stage(0);
-  if (kABufs == 2 && nsteps > 1) {
-#pragma unroll
-    for (int q = 0; q < kLoads; ++q) av[q] = *reinterpret_cast<const u32x4*>(arow[q] + kStep);
-  }
+  if (kABufs == 2 && nsteps > 1) load_av(1);
 
   f32x4 acc[2][NTC];
 #pragma unroll
@@ -761,7 +841,10 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
         for (int grp = 0; grp < 2; ++grp) {
           const uint8_t* slot = reinterpret_cast<const uint8_t*>(w_lds) + (wave * 2 + grp) * kGB +
                                 4 * kPitchDw * n;
-          if (sp == 0)  // k even: the step starts at a dword; odd: 2 bytes in (kSB is 2 mod 4)
+          if constexpr (kDwords)
+            dword_fields<KIND>(slot, (uint32_t)(k * kSB) - dword_first<KIND>(k, p.row_bytes),
+                               PART && k == nsteps - 1 ? min(g, last_pairs - 1) : g, f[grp]);
+          else if (sp == 0)  // k even: the step starts at a dword; odd: 2 bytes in (kSB is 2 mod 4)
             lds_fields<KIND, 0>(slot, g, f[grp]);
           else
             lds_fields<KIND, 2>(slot, g, f[grp]);
@@ -770,10 +853,7 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
           stage(k + 1);
         }
-        if (k + kABufs < nsteps) {
-#pragma unroll
-          for (int q = 0; q < kLoads; ++q) av[q] = *reinterpret_cast<const u32x4*>(arow[q] + (k + kABufs) * kStep);
-        }
+        if (k + kABufs < nsteps) load_av(k + kABufs);
         if constexpr (kABufs == 1) lds_barrier();  // every wave's activations of step k are written
         const f16* ab = a_lds + (kABufs == 2 ? sp * kABuf : 0);
 
@@ -839,11 +919,11 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
   write_chunk<MODE, OT, NTC>(p, acc, t0, g, row0, row1);
 }
 
-// PART (rows that end within a step) takes the unstaged body.
+// PART (rows that end within a step): the unstaged body, or the dword types' staged one.
 template <int KIND, int MODE, typename OT, int WAVES, int NT, bool STAGED, bool PART>
-__global__ __launch_bounds__(64 * WAVES, kMinWaves) void prompt_kernel(PromptParams p) {
+__global__ __launch_bounds__(64 * WAVES, kMinWaves<KIND>) void prompt_kernel(PromptParams p) {
   constexpr int kThreadsWg = 64 * WAVES;
-  constexpr bool kStagedHere = STAGED && !PART && kStagedKind<KIND>;
+  constexpr bool kStagedHere = STAGED && kStagedKind<KIND> && (!PART || kDwordRows<KIND>);
   __shared__ __attribute__((aligned(16))) uint8_t w_lds[kStagedHere ? WAVES * 2 * kGroupBytes<KIND> : 16];
   __shared__ DirectTables<KIND> tab;
   __shared__ __attribute__((aligned(16))) f16 a_lds[(kStagedHere ? activation_buffers<NT>() : 1) * NT * 16 * kSlotCols<KIND>];
@@ -919,7 +999,7 @@ __global__ __launch_bounds__(64 * WAVES, kMinWaves) void prompt_kernel(PromptPar
     constexpr int NTC = decltype(ntc)::value;
     if constexpr (NTC <= NT) {
       if constexpr (kStagedHere)
-        run_chunk_staged<KIND, MODE, OT, WAVES, NT, NTC>(p, tab, a_lds, w_lds, e, t0, rb, tid, wave);
+        run_chunk_staged<KIND, MODE, OT, WAVES, NT, NTC, PART>(p, tab, a_lds, w_lds, e, t0, rb, tid, wave);
       else
         run_chunk<KIND, MODE, OT, WAVES, NTC, PART>(p, tab, a_lds, e, t0, rb, tid, wave);
     }
@@ -973,12 +1053,25 @@ int launch_prompt(PromptParams& p, hipStream_t s) {
   // staged rows read whole dwords: the stacks' bases and a row's bytes multiples of 4
   const bool aligned = ((uintptr_t)p.blocks[0] & 3) == 0 && ((uintptr_t)p.blocks[1] & 3) == 0 &&
                        p.row_bytes % 4 == 0 && p.mat_bytes % 4 == 0;
+  // the dword types: whole groups of rows a wave, rows of a slot or more
+  const bool whole = p.rows % (MODE == PM_GLU ? 16 : 32) == 0 && p.row_bytes >= 4 * kSlotDwords<KIND>;
+  const bool staged = kStaged && kStagedKind<KIND> && aligned && (!kDwordRows<KIND> || whole);
   if (p.cols % kStep != 0) {
-    if constexpr (kMayPart<KIND>) go(std::false_type(), std::true_type());
-    else return STRATA_ERR_SHAPE;
+    if constexpr (kMayPart<KIND>) {
+      if constexpr (kDwordRows<KIND>) {
+        if (staged) {
+          go(std::true_type(), std::true_type());
+          STRATA_CHECK_LAUNCH();
+          return STRATA_OK;
+        }
+      }
+      go(std::false_type(), std::true_type());
+    } else {
+      return STRATA_ERR_SHAPE;
+    }
   } else {
-    if constexpr (kStaged && kStagedKind<KIND>) {
-      if (aligned) {
+    if constexpr (kStagedKind<KIND>) {
+      if (staged) {
         go(std::true_type(), std::false_type());
         STRATA_CHECK_LAUNCH();
         return STRATA_OK;

@@ -368,7 +368,7 @@ int launch_prompt_wide(PromptParams& p, hipStream_t s) {
 // form (skip_full); otherwise the chunked form alone.
 template <int KIND, int MODE, typename OT>
 int launch_prompt_split(PromptParams& p, hipStream_t s) {
-  if constexpr (kStagedKind<KIND>) {  // the types the wide form decodes
+  if constexpr (kStagedKind<KIND> && !kDwordRows<KIND>) {  // the types the wide form decodes
     if (wide_takes<MODE>(p)) {
       const int rc = launch_prompt_wide<KIND, MODE, OT>(p, s);
       if (rc) return rc;

@@ -71,6 +71,20 @@ __device__ __forceinline__ uint32_t split_sum(float s) {
   return hi | (half_of(v - half_bits_to_f32(hi)) << 16);
 }
 
+// The mins' side of a step's min product: lane (n, g)'s two runs' mins of row n, against their sums' two parts each.
+template <int KIND>
+__device__ __forceinline__ f16x8 own_mins(const RunPair<KIND>& f, int g) {
+  uint32_t mn[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int sb = 2 * g + h, tb = 8 * (sb & 3);
+    const uint32_t b1 = (f.sm[1] >> tb) & 255, b2 = (f.sm[2] >> tb) & 255;
+    const uint32_t v = sb >= 4 ? ((b2 >> 4) | ((b1 >> 6) << 4)) : (b1 & 63);
+    mn[h] = __builtin_bit_cast(uint32_t, strata_prompt::both((int)v));
+  }
+  return __builtin_bit_cast(f16x8, u32x4{mn[0], mn[1], 0u, 0u});
+}
+
 template <int KIND>
 constexpr bool kStagedRows = KIND == K_Q4_K || KIND == K_Q6_K || KIND == K_Q8_0;
 // 16-byte pieces of a wave's part of a row, from the aligned one that holds its first byte (an even one), and the pitch
@@ -98,16 +112,6 @@ __device__ __forceinline__ void dma_x4(const uint8_t* base, uint32_t voff, uint3
                  : "memory");
 }
 
-// N words at an even byte offset of LDS: N + 1 aligned dwords, shifted
-template <int N>
-__device__ __forceinline__ void words_at(const uint8_t* base, uint32_t off, uint32_t (&w)[N]) {
-  uint32_t d[N + 1];
-#pragma unroll
-  for (int k = 0; k <= N; ++k) d[k] = strata_prompt::lds_at<uint32_t>(base, (off & ~3u) + 4u * k);
-#pragma unroll
-  for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_alignbyte(d[k + 1], d[k], off & 3u);
-}
-
 // run pair g's fields of a step that starts at byte `off` of LDS (the types of 16-byte steps: a multiple of 16)
 template <int KIND>
 __device__ __forceinline__ void staged_fields(const uint8_t* lds, uint32_t off, int g, RunPair<KIND>& f) {
@@ -118,31 +122,8 @@ __device__ __forceinline__ void staged_fields(const uint8_t* lds, uint32_t off, 
     f.sm = u32x4{h[1], h[2], h[3], 0u};
 #pragma unroll
     for (int i = 0; i < 2; ++i) f.qs[i] = strata_prompt::lds_at<u32x4a>(lds, off + 16 + 32 * g + 16 * i);
-  } else if constexpr (KIND == K_Q8_0) {  // 68 bytes: d, 32 codes, d, 32 codes
-    uint32_t w[17];
-#pragma unroll
-    for (int k = 0; k < 17; ++k) w[k] = strata_prompt::lds_at<uint32_t>(lds, off + 68 * g + 4 * k);
-    f.d[0] = (uint16_t)(w[0] & 0xffffu);
-    f.d[1] = (uint16_t)(w[8] >> 16);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      f.q[k / 4][k % 4] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
-      f.q[2 + k / 4][k % 4] = w[9 + k];
-    }
   } else {
-    static_assert(KIND == K_Q6_K, "the staged types");
-    const LaneOffsets<K_Q6_K> o = strata_mv::lane_offsets<K_Q6_K>(g);
-    uint32_t ql[8], qh[8];
-    words_at<8>(lds, off + o.qs, ql);
-    words_at<8>(lds, off + o.a, qh);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      f.ql[k / 4][k % 4] = ql[k];
-      f.qh[k / 4][k % 4] = qh[k];
-    }
-    f.sc[0] = strata_prompt::lds_at<uint16_t>(lds, off + o.b);
-    f.sc[1] = strata_prompt::lds_at<uint16_t>(lds, off + o.b + 4);
-    f.d = strata_prompt::lds_at<uint16_t>(lds, off + o.d);
+    strata_prompt::dword_fields<KIND>(lds, off, g, f);
   }
 }
 
@@ -349,18 +330,9 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(d, part[j], acc[j]);
       if constexpr (kHasMin<KIND>) {
-        uint32_t mn[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int sb = 2 * g + h, tb = 8 * (sb & 3);
-          const uint32_t b1 = (f[s].sm[1] >> tb) & 255, b2 = (f[s].sm[2] >> tb) & 255;
-          const uint32_t v = sb >= 4 ? ((b2 >> 4) | ((b1 >> 6) << 4)) : (b1 & 63);
-          mn[h] = __builtin_bit_cast(uint32_t, strata_prompt::both((int)v));  // against the high and the low part
-        }
         const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
         const f32x4 mm = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(f16x8, u32x4{sums[s][0], sums[s][1], 0u, 0u}),
-            __builtin_bit_cast(f16x8, u32x4{mn[0], mn[1], 0u, 0u}), z, 0, 0, 0);
+            __builtin_bit_cast(f16x8, u32x4{sums[s][0], sums[s][1], 0u, 0u}), own_mins<KIND>(f[s], g), z, 0, 0, 0);
         const float dm = strata_prompt::kSumScale * strata_mv::half_bits(f[s].dd >> 16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(-dm, mm[j], acc[j]);

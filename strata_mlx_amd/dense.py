@@ -23,6 +23,7 @@ from . import blocks as B
 MAX_TOKENS = 8  # more than a window: a chunk of a prompt, multiplied as floats (dense.py:33)
 # the same for 16-bit tokens and rows of at most WINDOW_COLS inputs: what the MFMA window kernel takes in one pass
 WINDOW_TOKENS, WINDOW_COLS = 16, 4096
+CHUNK_TOKENS = 1 << 30  # tokens up to which a longer 16-bit chunk is multiplied straight from the blocks
 # Q3_K layers held as planes (blocks.q3k_planes), as the reference holds them (dense.py:190, 214-215), when True;
 # by default they stay the file's blocks, which the register decode reads at twice the planes window's speed
 PLANES = False
@@ -65,6 +66,11 @@ class BlockLinear:
         if kind == "Q3_K" and PLANES:  # held as planes instead: aligned words for the window kernel
             self.planes, self.blocks = B.q3k_planes(blocks, *shape), None
 
+    def _chunk_takes(self) -> bool:
+        cols = self.input_dims
+        return (self.kind not in B.NO_GRID and cols % (64 if B.block_weights(self.kind) < 256 else 256) == 0
+                and self.output_dims * B.row_bytes(self.kind, cols) < 1 << 32)
+
     @property
     def nbytes(self) -> int:
         if self.planes is not None:
@@ -98,6 +104,8 @@ class BlockLinear:
                 tokens <= WINDOW_TOKENS and cols <= WINDOW_COLS and x2.dtype != torch.float32
                 and cols % (64 if B.block_weights(self.kind) < 256 else 256) == 0):
             out = B.window_matvec(self.blocks, self.kind, rows, cols, x2, row_ids=row_ids)
+        elif x2.dtype in (torch.float16, torch.bfloat16) and tokens <= CHUNK_TOKENS and self._chunk_takes():
+            out = B.chunk_matmul(self.blocks, self.kind, rows, cols, x2)
         elif x2.dtype in (torch.float16, torch.bfloat16):
             out = float16_chunk(self.floats(torch.float16), x2)
         elif B.tileable(self.kind, rows, cols):
