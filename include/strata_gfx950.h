@@ -198,6 +198,15 @@ int strata_rows_to_f16_sums(const void* a, int64_t rows, int64_t cols, int a_dty
 int strata_rows_from_f32(const float* c, int64_t rows, int64_t cols, const uint32_t* row_max, int out_dtype,
                          void* out, void* stream);
 
+/* out[t, r] = W[r, :] . x[t, :] for a chunk of `tokens` rows of x (dtype F16 or BF16), out (tokens, rows) in the same
+ * type: on MFMA straight from the blocks, weights rounded to float16 (exact where 11 bits hold a type's integers),
+ * float32 sums. cols as strata_tiles_gate_up_swiglu's; a matrix below 4 GiB. x at a 16-byte boundary. workspace:
+ * strata_dense_chunk_workspace(tokens, cols) bytes at a 16-byte boundary, written by the call.
+ * Replaces the product of strata_mlx/dense.py:234-242 for chunks too short to be worth unpacking a layer. */
+int64_t strata_dense_chunk_workspace(int64_t tokens, int64_t cols);
+int strata_dense_chunk(int kind, const void* blocks, int64_t rows, int64_t cols, const void* x, int64_t tokens,
+                       int dtype, void* out, void* workspace, void* stream);
+
 /* strata_route_tiles with its workspace in the library's own device memory (a file-scope array of about 1 MB a
  * GPU, held until the process ends): the call allocates nothing, for callers that cannot allocate (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. pairs at

@@ -120,19 +120,21 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
   __shared__ __attribute__((aligned(16))) uint8_t slots[STAGED ? kMaxWaves * RG * kGB : 16];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
-  const int r0 = blockIdx.x * 16 * RG, tile0 = blockIdx.y * NT;
+  const int row_blocks = (p.rows + 16 * RG - 1) / (16 * RG), tile0 = blockIdx.y * NT;
   const int last_tile = (p.tokens + 15) / 16 - 1;
 
   const int last_pairs = kMayPart<KIND> ? (p.cols - (p.nsteps - 1) * kStep) / 64 : 4;
   const uint32_t back = (uint32_t)max(0, g - (last_pairs - 1)) * (kStepBytes<KIND> / 4);  // in a partial last step
   const LaneOffsets<KIND> o = strata_mv::lane_offsets<KIND>(g);
-  uint32_t off[RG];
-#pragma unroll
-  for (int i = 0; i < RG; ++i) off[i] = (uint32_t)min(r0 + 16 * i + n, p.rows - 1) * (uint32_t)p.row_bytes;
-  auto load = [&](int k, RunPair<KIND>(&f)[RG]) {
+  // row block rb's first row as a base; rows past the last block's are the matrix's last row
+  auto block_at = [&](int rb) { return p.blocks + (int64_t)rb * (16 * RG) * p.row_bytes; };
+  auto load = [&](int rb, int k, RunPair<KIND>(&f)[RG]) {
     const uint32_t at = (uint32_t)k * kStepBytes<KIND> - (kMayPart<KIND> && k == p.nsteps - 1 ? back : 0u);
 #pragma unroll
-    for (int i = 0; i < RG; ++i) strata_mv::load_fields<KIND>(p.blocks, off[i] + at, o, f[i]);
+    for (int i = 0; i < RG; ++i) {
+      const int row = min(16 * i + n, p.rows - 1 - rb * (16 * RG));
+      strata_mv::load_fields<KIND>(block_at(rb), (uint32_t)row * (uint32_t)p.row_bytes + at, o, f[i]);
+    }
   };
   uint32_t voff[RG][kGL];
   const uint32_t slot0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)slots + (uint32_t)(wave * RG * kGB));
@@ -143,15 +145,27 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
 #pragma unroll
       for (int l = 0; l < kGL; ++l) {
         const int c = 64 * l + lane, q = min(c / kPitchDw, 15), d = min(c % kPitchDw, strata_prompt::kSlotDwords<KIND> - 1);
-        voff[r][l] = (uint32_t)min(r0 + 16 * r + q, p.rows - 1) * (uint32_t)p.row_bytes + 4u * (uint32_t)d;
+        voff[r][l] = (uint32_t)(16 * r + q) * (uint32_t)p.row_bytes + 4u * (uint32_t)d;
       }
   }
-  auto stage = [&](int k) {
-    const uint8_t* base = p.blocks + strata_prompt::dword_first<KIND>(k, p.row_bytes);
+  auto stage = [&](int rb, int k) {
+    const uint8_t* base = block_at(rb) + strata_prompt::dword_first<KIND>(k, p.row_bytes);
+    const int last = p.rows - 1 - rb * (16 * RG);  // the block's last row
+    if (last < 16 * RG - 1) {
 #pragma unroll
-    for (int r = 0; r < RG; ++r)
+      for (int r = 0; r < RG; ++r)
 #pragma unroll
-      for (int l = 0; l < kGL; ++l) strata_prompt::dma_dword(base, voff[r][l], slot0 + (uint32_t)(r * kGB + 256 * l));
+        for (int l = 0; l < kGL; ++l) {
+          const int q = 16 * r + min((64 * l + lane) / strata_prompt::kSlotPitch<KIND>, 15);
+          strata_prompt::dma_dword(base, voff[r][l] - (uint32_t)max(0, q - last) * (uint32_t)p.row_bytes,
+                                   slot0 + (uint32_t)(r * kGB + 256 * l));
+        }
+    } else {
+#pragma unroll
+      for (int r = 0; r < RG; ++r)
+#pragma unroll
+        for (int l = 0; l < kGL; ++l) strata_prompt::dma_dword(base, voff[r][l], slot0 + (uint32_t)(r * kGB + 256 * l));
+    }
   };
   const u32x4* at[NT];  // tile i's operands of step 0 (past the last tile: the last again, written nowhere)
   const u32x2* sat[NT];
@@ -166,12 +180,12 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
 #pragma unroll
     for (int i = 0; i < NT; ++i) dst[i] = at[i][(k * 8 + m) * 64];
   };
-  int k = wave;
+  int k = wave, rb = blockIdx.x;
   RunPair<KIND> f[RG];
   if constexpr (STAGED)
-    stage(k);
+    stage(rb, k);
   else
-    load(k, f);
+    load(rb, k, f);
 #pragma unroll
   for (int m = 0; m < kAhead; ++m) load_a(k, m, a[m]);
   for (int i = tid; i < 256; i += blockDim.x) {  // the tables
@@ -179,6 +193,28 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
     strata_mv::fetch_tables<KIND>(tf, i);
     strata_mv::store_tables<KIND>(tab, tf, i);
   }
+  auto write = [&](int b) {
+    for (int c = wave; c < RG * NT; c += waves) {  // one (row group, tile) a wave: lane (n, g) row n, tokens 4 g + j
+      f32x4 t = red[0][c][lane];
+#pragma unroll
+      for (int w = 1; w < kMaxWaves; ++w) {
+        if (w < waves) {
+          const f32x4 v = red[w][c][lane];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) t[j] += v[j];
+        }
+      }
+      const int row = b * (16 * RG) + 16 * (c / NT) + n;
+      if (row >= p.rows) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int token = (tile0 + c % NT) * 16 + 4 * g + j;
+        if (token >= p.tokens) continue;
+        const float v = p.a_max != nullptr ? __builtin_ldexpf(t[j], row_exponent(p.a_max[token])) : t[j];
+        reinterpret_cast<OT*>(p.out)[(int64_t)token * p.rows + row] = from_f32<OT>(v);
+      }
+    }
+  };
   f32x4 acc[RG][NT];
 #pragma unroll
   for (int r = 0; r < RG; ++r)
@@ -186,8 +222,11 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
     for (int i = 0; i < NT; ++i) acc[r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   strata_prompt::lds_barrier();  // the tables are written; the loads stay in flight
 
-  for (; k < p.nsteps; k += waves) {
-    const int next = k + waves < p.nsteps ? k + waves : k;
+  for (;;) {
+    // the wave's next step: of this row block, or the first of the workgroup's next one
+    const bool done = k + waves >= p.nsteps;
+    const int next = done ? wave : k + waves, nrb = done ? rb + gridDim.x : rb;
+    const bool more = nrb < row_blocks;
     RunPair<KIND> fn[STAGED ? 1 : RG];
     if constexpr (STAGED) {
       strata_prompt::wait_loads();
@@ -197,12 +236,12 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
       for (int r = 0; r < RG; ++r)
         strata_prompt::dword_fields<KIND>(slots + (wave * RG + r) * kGB + 4 * strata_prompt::kSlotPitch<KIND> * n, off,
                                           gl, f[r]);
-      if (next != k) {
+      if (more) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        stage(next);
+        stage(nrb, next);
       }
     } else {
-      load(next, fn);
+      load(more ? nrb : rb, next, fn);
     }
     f32x4 part[RG][NT];
 #pragma unroll
@@ -252,32 +291,21 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void chunk_kernel(ChunkParams p)
 #pragma unroll
       for (int r = 0; r < RG; ++r) f[r] = fn[r];
     }
-  }
-
+    if (done) {  // the row block's sums: the waves' parts meet in LDS
+      if (rb != (int)blockIdx.x) strata_prompt::lds_barrier();  // the last block's parts have been read
 #pragma unroll
-  for (int r = 0; r < RG; ++r)
+      for (int r = 0; r < RG; ++r)
 #pragma unroll
-    for (int i = 0; i < NT; ++i) red[wave][r * NT + i][lane] = acc[r][i];
-  __syncthreads();
-  for (int c = wave; c < RG * NT; c += waves) {  // one (row group, tile) a wave: lane (n, g) row n, tokens 4 g + j
-    f32x4 t = red[0][c][lane];
-#pragma unroll
-    for (int w = 1; w < kMaxWaves; ++w) {
-      if (w < waves) {
-        const f32x4 v = red[w][c][lane];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] += v[j];
-      }
+        for (int i = 0; i < NT; ++i) {
+          red[wave][r * NT + i][lane] = acc[r][i];
+          acc[r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      strata_prompt::lds_barrier();
+      write(rb);
+      if (!more) break;
     }
-    const int row = r0 + 16 * (c / NT) + n;
-    if (row >= p.rows) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int token = (tile0 + c % NT) * 16 + 4 * g + j;
-      if (token >= p.tokens) continue;
-      const float v = p.a_max != nullptr ? __builtin_ldexpf(t[j], row_exponent(p.a_max[token])) : t[j];
-      reinterpret_cast<OT*>(p.out)[(int64_t)token * p.rows + row] = from_f32<OT>(v);
-    }
+    k = next;
+    rb = nrb;
   }
 }
 
@@ -314,7 +342,9 @@ int launch_chunk(ChunkParams& p, const void* x, void* workspace, hipStream_t s) 
                       p.row_bytes >= 4 * strata_prompt::kSlotDwords<KIND>;
   auto go = [&](auto rg, auto ntc) {
     constexpr int RG = decltype(rg)::value, NT = decltype(ntc)::value;
-    const dim3 grid((unsigned)((p.rows + 16 * RG - 1) / (16 * RG)), (unsigned)token_blocks);
+    // one workgroup a CU, which goes on to its next row block: its rows are asked for before the last one's sums meet
+    const int blocks_x = (p.rows + 16 * RG - 1) / (16 * RG);
+    const dim3 grid((unsigned)min(blocks_x, max(1, strata_mv::device_cus() / token_blocks)), (unsigned)token_blocks);
     if constexpr (strata_prompt::kDwordRows<KIND>) {
       if (staged) {
         hipLaunchKernelGGL((chunk_kernel<KIND, OT, RG, NT, true>), grid, block, 0, s, p);

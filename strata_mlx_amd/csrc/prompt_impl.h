@@ -4,8 +4,8 @@
 //
 // The types decoded by byte arithmetic (decode_linear4) fold their integer scales in too, so that what is left for
 // the sums is one d a 256-weight block; Q4_K and Q5_K add one MFMA a step for their mins. A layer of 256 Q4_K / Q6_K
-// experts at 384 tokens (1536 x 4096, top-8, bfloat16): 1370 us a launch of gate or up through the decode of float32
-// weights into LDS (gemm_impl.h) -> 764 us for both with the SwiGLU; down 1290 -> 684 us.
+// experts at 384 tokens (1536 x 4096, top-8, bfloat16): 1370 us a launch of gate or up and 1290 us of down through the
+// decode of float32 weights into LDS (gemm_impl.h); here the whole layer takes 995 us.
 //
 // c[s, :] = W[e(s)] . a[s, :]. A workgroup (4 waves) takes a chunk, up to NT = 3 consecutive tiles of one expert
 // (a run of one expert's tiles is cut into chunks of NT from its first tile; the workgroup at a chunk's first tile
@@ -377,6 +377,28 @@ __device__ __forceinline__ void write_chunk(const PromptParams& p, const f32x4 (
   }
 }
 
+// The step's min products taken off the sums: the mins of the lane's two rows (groups f[0], f[1]) times each slot's sums
+// of activations, which lie behind its columns in LDS.
+template <int KIND, int NTC>
+__device__ __forceinline__ void take_mins(const RunPair<KIND> (&f)[2], const f16* a_lds, int n, int g,
+                                          f32x4 (&acc)[2][NTC]) {
+  const f16x8 b0 = min_operand<KIND>(f[0], g), b1 = min_operand<KIND>(f[1], g);
+  const float m0 = kSumScale * strata_mv::half_bits(f[0].dd >> 16);
+  const float m1 = kSumScale * strata_mv::half_bits(f[1].dd >> 16);
+#pragma unroll
+  for (int i = 0; i < NTC; ++i) {
+    const f16x8 as = *reinterpret_cast<const f16x8*>(a_lds + (i * 16 + n) * kSlotCols<KIND> + kStep + 8 * (g & 1));
+    const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4 q0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b0, z, 0, 0, 0);
+    const f32x4 q1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b1, z, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc[0][i][j] = __builtin_fmaf(-m0, q0[j], acc[0][i][j]);
+      acc[1][i][j] = __builtin_fmaf(-m1, q1[j], acc[1][i][j]);
+    }
+  }
+}
+
 // One chunk of exactly NTC tiles (NTC at compile time: no per-tile branches between the MFMAs).
 // PART: the rows end within a step (kMayPart): in the last one, lanes past the row's run pairs take its last run pair
 // again and the activations past the row are zeros.
@@ -521,23 +543,7 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
             for (int q = 0; q < 4; ++q) mfma_group(a8[q], w0 + 4 * q, w1 + 4 * q);
           }
         }
-        if constexpr (kHasMin<KIND>) {
-          const f16x8 b0 = min_operand<KIND>(f[sp][0], g), b1 = min_operand<KIND>(f[sp][1], g);
-          const float m0 = kSumScale * strata_mv::half_bits(f[sp][0].dd >> 16);
-          const float m1 = kSumScale * strata_mv::half_bits(f[sp][1].dd >> 16);
-#pragma unroll
-          for (int i = 0; i < NTC; ++i) {
-            const f16x8 as = *reinterpret_cast<const f16x8*>(a_lds + (i * 16 + n) * kP + kStep + 8 * (g & 1));
-            const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
-            const f32x4 q0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b0, z, 0, 0, 0);
-            const f32x4 q1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, b1, z, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              acc[0][i][j] = __builtin_fmaf(-m0, q0[j], acc[0][i][j]);
-              acc[1][i][j] = __builtin_fmaf(-m1, q1[j], acc[1][i][j]);
-            }
-          }
-        }
+        if constexpr (kHasMin<KIND>) take_mins<KIND, NTC>(f[sp], a_lds, n, g, acc);
         if constexpr (has_step_scale<KIND>()) {
           const float s0 = step_scale<KIND>(f[sp][0]), s1 = step_scale<KIND>(f[sp][1]);
 #pragma unroll
@@ -581,16 +587,17 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
 // on a CU; at two (a third row buffer, or the IQ3_XXS codebook with its signs folded in, 32 KB) or at four (128
 // registers, spilled) the kernel ran slower.
 //
-// Q6_K, IQ4_NL, Q4_0 and Q8_0 rows too (kDwordRows), whose fields lie at 2 or 4 bytes past a boundary: loaded straight
-// into registers, their 16-byte loads ran several times longer than aligned ones. Their slots are an odd number of
+// Q4_K, Q5_K, Q6_K, IQ4_NL, Q4_0 and Q8_0 rows too (kDwordRows): loaded straight into registers, the 16-byte loads of
+// those whose fields lie 2 or 4 bytes past a boundary ran several times longer still. Their slots are an odd number of
 // dwords apart, so that reads of one dword spread over the banks, and each field is put together from dwords. Down of
-// a layer of 256 Q6_K experts at 384 tokens 684 -> DOWN_Q6K us.
+// a layer of 256 Q6_K experts at 384 tokens 684 -> 402 us (33 spilled registers less at two waves a SIMD among it),
+// gate and up in Q4_K 764 -> 600.
 template <int KIND>
-constexpr bool kDwordRows = KIND == K_Q6_K || KIND == K_IQ4_NL || KIND == K_Q4_0 || KIND == K_Q8_0;
+constexpr bool kDwordRows = KIND == K_Q4_K || KIND == K_Q5_K || KIND == K_Q6_K || KIND == K_IQ4_NL || KIND == K_Q4_0 || KIND == K_Q8_0;
 template <int KIND>
 constexpr bool kStagedKind = KIND == K_IQ3_S || KIND == K_IQ3_XXS || KIND == K_Q2_0 || kDwordRows<KIND>;
 template <int KIND>
-constexpr int kSlotDwords = (kStepBytes<KIND> + 2) / 4;  // dwords a row's step spans: 28, 25, 18; 53, 36, 36, 68
+constexpr int kSlotDwords = (kStepBytes<KIND> + 2) / 4;  // dwords a row's step spans: 28, 25, 18; Q6_K 53
 template <int KIND>
 constexpr int kSlotPitch = kDwordRows<KIND> ? kSlotDwords<KIND> | 1 : KIND == K_Q2_0 ? 20 : 28;  // dwords a row's slot
 template <int KIND>
@@ -675,7 +682,16 @@ __device__ __forceinline__ void words_at(const uint8_t* base, uint32_t off, uint
 // run pair g's fields of a step that starts at byte `off` of LDS (Q6_K: even; the others a multiple of 4)
 template <int KIND>
 __device__ __forceinline__ void dword_fields(const uint8_t* lds, uint32_t off, int g, RunPair<KIND>& f) {
-  if constexpr (KIND == K_Q6_K) {
+  if constexpr (KIND == K_Q4_K || KIND == K_Q5_K) {  // d, dmin, the 12 scale bytes, (Q5_K: 32 high-bit bytes,) codes
+    f.dd = lds_at<uint32_t>(lds, off);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) f.sm[k] = lds_at<uint32_t>(lds, off + 4 + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if constexpr (KIND == K_Q5_K) f.qh[k / 4][k % 4] = lds_at<uint32_t>(lds, off + 16 + 4 * k);
+      f.qs[k / 4][k % 4] = lds_at<uint32_t>(lds, off + (KIND == K_Q5_K ? 48 : 16) + 32 * g + 4 * k);
+    }
+  } else if constexpr (KIND == K_Q6_K) {
     const LaneOffsets<K_Q6_K> o = strata_mv::lane_offsets<K_Q6_K>(g);
     uint32_t ql[8], qh[8];
     words_at<8>(lds, off + o.qs, ql);
@@ -741,7 +757,8 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
   constexpr bool kDwords = kDwordRows<KIND>;
   constexpr int kSB = kStepBytes<KIND>, kDW = kSlotDwords<KIND>, kGL = kGroupLoads<KIND>, kPitchDw = kSlotPitch<KIND>;
   constexpr int kGB = kGroupBytes<KIND>;
-  constexpr int kABuf = NT * 16 * kPitch;  // float16: an activation buffer
+  constexpr int kP = kSlotCols<KIND>;
+  constexpr int kABuf = NT * 16 * kP;  // float16: an activation buffer
   constexpr int kABufs = activation_buffers<NT>();
   const int lane = tid & 63;
 
@@ -790,7 +807,7 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
     const int slot = (t0 + i) * 16 + m;
     const uint32_t r = p.a_row ? p.a_row[slot] : (uint32_t)slot;
     arow[q] = p.a + (int64_t)r * p.cols + 8 * piece;
-    adst[q] = (i * 16 + m) * kPitch + 8 * piece;
+    adst[q] = (i * 16 + m) * kP + 8 * piece;
   }
   u32x4 av[kLoads];
   auto load_av = [&](int k) {
@@ -805,6 +822,19 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
       }
     }
   };
+  // the types with mins: threads 0 .. 32 NTC - 1 bring a slot's 8 high or low sums of the step
+  static_assert(!kHasMin<KIND> || kABufs == 1, "one buffer");
+  const f16* srow = nullptr;
+  int sdst = 0;
+  u32x4 sv;
+  if constexpr (kHasMin<KIND>) {
+    const int c = min(tid, 32 * NTC - 1), m = c / 2, part = c % 2;
+    const int slot = t0 * 16 + m;
+    const uint32_t r = p.a_row ? p.a_row[slot] : (uint32_t)slot;
+    srow = p.a_sum + (int64_t)r * (nsteps * kSumCols) + 8 * part;
+    sdst = m * kP + kStep + 8 * part;
+    sv = *reinterpret_cast<const u32x4*>(srow);
+  }
   load_av(0);
   if constexpr (kABufs == 2) {
 #pragma unroll
@@ -835,6 +865,9 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
         } else {
 #pragma unroll
           for (int q = 0; q < kLoads; ++q) *reinterpret_cast<u32x4*>(a_lds + adst[q]) = av[q];
+          if constexpr (kHasMin<KIND>) {
+            if (tid < 32 * NTC) *reinterpret_cast<u32x4*>(a_lds + sdst) = sv;
+          }
         }
         RunPair<KIND> f[2];
 #pragma unroll
@@ -853,7 +886,10 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
           stage(k + 1);
         }
-        if (k + kABufs < nsteps) load_av(k + kABufs);
+        if (k + kABufs < nsteps) {
+          load_av(k + kABufs);
+          if constexpr (kHasMin<KIND>) sv = *reinterpret_cast<const u32x4*>(srow + (k + kABufs) * kSumCols);
+        }
         if constexpr (kABufs == 1) lds_barrier();  // every wave's activations of step k are written
         const f16* ab = a_lds + (kABufs == 2 ? sp * kABuf : 0);
 
@@ -868,7 +904,7 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
         auto read_a = [&](f16x8 (&a8)[4][NTC], int h, int q) {
 #pragma unroll
           for (int i = 0; i < NTC; ++i)
-            a8[q][i] = *reinterpret_cast<const f16x8*>(ab + (i * 16 + n) * kPitch + a_col<KIND>(g, h, q));
+            a8[q][i] = *reinterpret_cast<const f16x8*>(ab + (i * 16 + n) * kP + a_col<KIND>(g, h, q));
         };
         auto mfma_group = [&](const f16x8 (&a8)[NTC], const uint32_t* w0, const uint32_t* w1) {
           const f16x8 b0 = __builtin_bit_cast(f16x8, u32x4{w0[0], w0[1], w0[2], w0[3]});
@@ -904,6 +940,7 @@ __device__ __forceinline__ void run_chunk_staged(const PromptParams& p, const Di
             for (int q = 0; q < 4; ++q) mfma_group(a8[q], w0 + 4 * q, w1 + 4 * q);
           }
         }
+        if constexpr (kHasMin<KIND>) take_mins<KIND, NTC>(f, ab, n, g, acc);
         const float s0 = step_scale<KIND>(f[0]), s1 = step_scale<KIND>(f[1]);
 #pragma unroll
         for (int i = 0; i < NTC; ++i) {

@@ -9,6 +9,7 @@
     BlockEmbedding rows of an embedding decoded when their tokens come (dense.py:245-258).
 
 Up to MAX_TOKENS tokens (WINDOW_TOKENS in 16 bits) a product is a window, each block decoded once for every token. A
+few more (CHUNK_TOKENS) of float16 or bfloat16 are multiplied on MFMA straight from the blocks. A
 longer chunk (a prompt's) of float16 or bfloat16 tokens is multiplied as the reference multiplies it
 (dense.py:234-241): the layer dequantized for the chunk (strata_dequantize, each weight exact in float32 and
 rounded once to float16) and let go, then a library product with float32 sums (torch.mm; 4-6 times the tile
@@ -23,7 +24,10 @@ from . import blocks as B
 MAX_TOKENS = 8  # more than a window: a chunk of a prompt, multiplied as floats (dense.py:33)
 # the same for 16-bit tokens and rows of at most WINDOW_COLS inputs: what the MFMA window kernel takes in one pass
 WINDOW_TOKENS, WINDOW_COLS = 16, 4096
-CHUNK_TOKENS = 1 << 30  # tokens up to which a longer 16-bit chunk is multiplied straight from the blocks
+# tokens up to which a longer 16-bit chunk is multiplied straight from the blocks (blocks.chunk_matmul), above by a
+# library product of the dequantized layer: Q4_K 4096 x 4096, bfloat16, 77 tokens 15 against 42 us, 256 29 against 45,
+# 384 49 against 48; Q6_K 12288 x 4096, 256 tokens 71 against 95, 384 124 against 103
+CHUNK_TOKENS = 256
 # Q3_K layers held as planes (blocks.q3k_planes), as the reference holds them (dense.py:190, 214-215), when True;
 # by default they stay the file's blocks, which the register decode reads at twice the planes window's speed
 PLANES = False
