@@ -30,12 +30,15 @@ DENSE = {"Q4_0": (32, 18), "Q5_0": (32, 22), "Q8_0": (32, 34), "Q4_K": (256, 144
 NO_GRID = ("IQ2_S", "IQ2_XS", "IQ2_XXS", "IQ1_M")
 
 TOKENS_TILE = 16  # slots of a tile (strata_mlx/blocks.py:581)
-# (token, expert) pairs from which float16 activations go through tiles (the reference: 1600, strata_mlx/blocks.py:580).
-# Below, each pair decodes its expert's rows again, above, an expert's rows are decoded once for 16 pairs: 8 tokens
-# of top-8 of 256 experts 130 us a pair at a time against 151 in tiles, 12 tokens 234 against 197, 48 tokens 1241
-# against 374 (IQ3_S, 1536 x 4096); Q4_K / Q6_K 267 against 235, 395 against 314, 2464 against 584.
-TILES_FROM = 65
-TILES_FROM_BF16 = 16  # bfloat16, whose matvec is the generic one: 2 tokens 160 against 97 us, 48 tokens 2021 against 394
+# (token, expert) pairs from which 16-bit activations go through tiles (the reference: 1600, strata_mlx/blocks.py:580).
+# Above, an expert's rows are decoded once for 16 pairs; below, the decode kernels have the lower fixed cost. 256 experts,
+# top-8, 1536 x 4096, Q4_K / Q6_K float16: 5 tokens 164 us against 181 in tiles, 6 tokens 189 against 183, 8 tokens 254
+# against 186, 48 tokens 2464 against 584; 512 experts of 640 x 2560, top-10, IQ3_XXS: 4 tokens 56 against 57, 6 tokens
+# 77 against 57.
+TILES_FROM = 48
+# the same where gate and up take the persistent or codebook decode kernels at 4096 inputs (IQ3_S, Q2_0; IQ3_XXS in
+# float16): IQ3_S 8 tokens 130 us against 137, 9 tokens 171 against 138
+TILES_FROM_DECODE = 65
 TILES_FROM_ANY = 1600  # what the fused tile kernels do not take (float32, ragged rows)
 MATVEC_GLU_UPTO = 1 << 16  # pairs for which down takes silu(gate) * up itself (the reference: 30)
 
@@ -604,7 +607,8 @@ def _tiles_from(dtype: torch.dtype, up, gate, down) -> int:
     table = LOOKUP_GLU and all(lookable(lin, dtype) for lin in (up, gate, down))
     if table or not (same and _prompt_fused(gate, dtype) and _prompt_fused(down, dtype)):
         return max(TILES_FROM, TILES_FROM_ANY)
-    return TILES_FROM_BF16 if dtype == torch.bfloat16 else TILES_FROM
+    decode = ("IQ3_S", "Q2_0") if dtype == torch.bfloat16 else ("IQ3_S", "IQ3_XXS", "Q2_0")
+    return max(TILES_FROM, TILES_FROM_DECODE) if gate.kind in decode and gate.input_dims == 4096 else TILES_FROM
 
 
 def switch_glu(x: torch.Tensor, indices: torch.Tensor, up: BlockSwitchLinear, gate: BlockSwitchLinear,
@@ -621,7 +625,7 @@ def switch_glu(x: torch.Tensor, indices: torch.Tensor, up: BlockSwitchLinear, ga
     k = indices.shape[-1] if indices.ndim else 1
     flat = indices.reshape(-1)
     xs = x.reshape(-1, x.shape[-1])
-    if flat.numel() >= min(TILES_FROM, TILES_FROM_BF16) and flat.numel() >= _tiles_from(x.dtype, up, gate, down) and \
+    if flat.numel() >= TILES_FROM and flat.numel() >= _tiles_from(x.dtype, up, gate, down) and \
             all(tileable(lin.kind, lin.output_dims, lin.input_dims) for lin in (up, gate, down)):
         return _tiled_glu(x, indices, up, gate, down)
     if LOOKUP_GLU and flat.numel() >= LOOKUP_FROM and all(lookable(lin, x.dtype) for lin in (up, gate, down)):

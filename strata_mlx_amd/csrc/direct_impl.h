@@ -1387,6 +1387,12 @@ int launch_matvec_any(MatvecParams& p, int x_dtype, int out_dtype, bool glu, int
                  : launch_direct<KIND, false, false>(p, one, grid_y, grid_z, s);
     }
   }
+  if constexpr (routed_kind(KIND)) {  // bfloat16 tokens in the persistent routed forms
+    if (x_dtype == DT_BF16 && out_dtype == DT_BF16 && !glu) {
+      if (p.glu_out != nullptr && grid_z == 2 && routed_glu_takes<KIND>(p)) return launch_routed_glu<KIND, bf16_t>(p, s);
+      if (p.glu_out == nullptr && grid_z == 1 && routed_down_takes<KIND>(p)) return launch_routed_down<KIND, bf16_t>(p, s);
+    }
+  }
   if constexpr (FastTraits<KIND>::supported) {
     if (x_dtype == DT_F16 && out_dtype == DT_F16 && p.row_ids == nullptr) {
       // one token a pass (four waves a SIMD) up to 64 routed pairs: most experts are named once, and the second

@@ -4,6 +4,7 @@
 #include "prompt_wide.h"
 #include "window_impl.h"
 #include "chunk_impl.h"
+#include "routed_window.h"
 
 #ifndef STRATA_KIND
 #error "STRATA_KIND must name a GGUF type id"
@@ -73,3 +74,13 @@ int STRATA_CAT(chunk_launch_, STRATA_KIND)(ChunkParams& p, const void* x, int dt
 }
 
 }  // namespace strata_chunk
+
+namespace strata_rwin {
+
+int STRATA_CAT(rwin_launch_, STRATA_KIND)(const RwinParams& p, int dtype, hipStream_t s) {
+  if (p.blocks[1] != nullptr)
+    return dtype == DT_F16 ? launch_rwin<STRATA_KIND, f16, 2>(p, s) : launch_rwin<STRATA_KIND, bf16_t, 2>(p, s);
+  return dtype == DT_F16 ? launch_rwin<STRATA_KIND, f16, 1>(p, s) : launch_rwin<STRATA_KIND, bf16_t, 1>(p, s);
+}
+
+}  // namespace strata_rwin

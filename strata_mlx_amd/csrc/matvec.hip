@@ -1,7 +1,7 @@
 // C-ABI entry points of the dequant and matvec family (declared in include/strata_gfx950.h).
 // Arguments are checked here; the kernels live in matvec_impl.h, one object per block type.
 #include "matvec_impl.h"
-#include "window_impl.h"
+#include "routed_window.h"
 
 namespace strata_mv {
 #define STRATA_DECLARE(K)                                                                                    \
@@ -39,9 +39,60 @@ STRATA_DECLARE(42)
 #undef STRATA_DECLARE
 }  // namespace strata_window
 
+namespace strata_rwin {
+#define STRATA_DECLARE(K) int rwin_launch_##K(const RwinParams&, int, hipStream_t);
+STRATA_DECLARE(2)
+STRATA_DECLARE(6)
+STRATA_DECLARE(8)
+STRATA_DECLARE(11)
+STRATA_DECLARE(12)
+STRATA_DECLARE(14)
+STRATA_DECLARE(18)
+STRATA_DECLARE(20)
+STRATA_DECLARE(21)
+STRATA_DECLARE(13)
+STRATA_DECLARE(23)
+STRATA_DECLARE(42)
+#undef STRATA_DECLARE
+}  // namespace strata_rwin
+
 using namespace strata_mv;
 
 namespace {
+
+int rwin_by_kind(int kind, const strata_rwin::RwinParams& p, int dtype, hipStream_t s) {
+  switch (kind) {
+#define STRATA_CASE(K) \
+  case K: return strata_rwin::rwin_launch_##K(p, dtype, s);
+    STRATA_CASE(2)
+    STRATA_CASE(6)
+    STRATA_CASE(8)
+    STRATA_CASE(11)
+    STRATA_CASE(12)
+    STRATA_CASE(14)
+    STRATA_CASE(18)
+    STRATA_CASE(20)
+    STRATA_CASE(21)
+    STRATA_CASE(13)
+    STRATA_CASE(23)
+    STRATA_CASE(42)
+#undef STRATA_CASE
+    default: return STRATA_ERR_KIND;
+  }
+}
+
+constexpr int kRoutedTokens = 8, kRoutedPairs = 80;
+
+// Routed products that go to rwin_kernel: those in bfloat16, whose other kernel is the generic matvec (a layer of
+// Q4_K / Q6_K experts at one token 115 -> 51 us, at four 342 -> 130), but for IQ3_S's and Q2_0's at up to eight tokens
+// in the shapes of the persistent routed forms, which take bfloat16 themselves (26 against 49 us at one token, 144
+// against 207 at eight). float16 stays on the matvecs, as fast or faster (Q4_K / Q6_K 36 against 49, 138 against 135).
+bool rwin_wanted(int kind, const MatvecParams& p, int dtype, bool with_h) {
+  if (dtype != DT_BF16) return false;
+  const bool routed = kind == K_IQ3_S || kind == K_Q2_0;
+  if (p.blocks[1] != nullptr) return !(with_h && routed && p.cols == 4096 && p.pairs / p.share <= kRoutedTokens);
+  return !(routed && (p.cols == 1536 || p.cols == 2560) && p.pairs <= kRoutedPairs);
+}
 
 constexpr int64_t kShortRows = 8192;
 constexpr int64_t kLongRows = 16384;  // above, one float16 token of Q8_0 takes the window kernel
@@ -170,6 +221,24 @@ int expert_common(int kind, const void* a, const void* b, int64_t experts, int64
   p.pairs = (int)pairs;
   p.share = (int)share;
   p.mode = MODE_EXPERT;
+  if (!glu && dtype != DT_F32 && rwin_wanted(kind, p, dtype, out_h != nullptr)) {
+    strata_rwin::RwinParams w = {};
+    w.blocks[0] = p.blocks[0];
+    w.blocks[1] = p.blocks[1];
+    w.idx = idx;
+    w.x = x;
+    w.out[0] = out_a;
+    w.out[1] = out_b;
+    w.h = out_h;
+    w.mat_bytes = p.mat_bytes;
+    w.experts = (uint32_t)experts;
+    w.rows = p.rows;
+    w.cols = p.cols;
+    w.row_bytes = p.row_bytes;
+    w.pairs = p.pairs;
+    w.share = p.share;
+    if (strata_rwin::rwin_takes(kind, w)) return rwin_by_kind(kind, w, dtype, (hipStream_t)stream);
+  }
   if (out_h != nullptr) {  // gate and up with silu(gate) * up: one launch where the float16 kernels take it
     p.glu_out = out_h;
     rc = launch_by_kind(kind, p, dtype, dtype, false, (int)pairs, 2, (hipStream_t)stream);
@@ -411,7 +480,7 @@ int strata_dense_matvec(int kind, const void* blocks, int64_t rows, int64_t cols
     w.cols = p.cols;
     w.row_bytes = p.row_bytes;
     w.tokens = p.tokens;
-    if (strata_window::window_takes(kind, w)) return window_by_kind(kind, w, x_dtype, (hipStream_t)stream);
+    if (strata_window::window_takes(kind, w, x_dtype == DT_F16)) return window_by_kind(kind, w, x_dtype, (hipStream_t)stream);
   }
   return launch_by_kind(kind, p, x_dtype, out_dtype, false, 1, 1, (hipStream_t)stream);
 }

@@ -186,6 +186,9 @@ __device__ __forceinline__ void fold_pairs(uint32_t (&w)[4], h2v m, uint32_t (&l
   }
 }
 
+// Element h of a pair of fields.
+__device__ __forceinline__ uint16_t pair_at(const uint16_t (&v)[2], int h) { return h ? v[1] : v[0]; }
+
 // decode_folded4 of the types without an IQ3 or Q2_0 codebook; SPLIT (kInexact): the weights as w + lo.
 template <int KIND, bool SPLIT = false>
 __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, int g, int l, uint32_t (&w)[4],
@@ -211,7 +214,7 @@ __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, in
     const uint32_t c0 = (h ? q0 : q0 << 4) & hi_nibbles, c1 = (h ? q1 : q1 << 4) & hi_nibbles;
     const uint32_t h0 = ((f.qh[l >> 1][2 * (l & 1)] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
     const uint32_t h1 = ((f.qh[l >> 1][2 * (l & 1) + 1] >> r2) & 0x03030303u) | 0x3C3C3C3Cu;
-    const int sc = (int8_t)(f.sc[h] >> (8 * (l >> 1)));  // a scale every 16 weights
+    const int sc = (int8_t)(pair_at(f.sc, h) >> (8 * (l >> 1)));  // a scale every 16 weights
     if constexpr (SPLIT) {  // the integers code - 32, then their products
       codes_folded(c0, c1, h0, h1, both(64), both(-96), w);
       fold_pairs<true>(w, both(sc), lo);
@@ -234,7 +237,7 @@ __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, in
     if constexpr (KIND == K_Q8_0) {
       strata_mv::bytes_to_h2<128>(f.q[2 * h + (l >> 1)][2 * (l & 1)] ^ 0x80808080u, w);
       strata_mv::bytes_to_h2<128>(f.q[2 * h + (l >> 1)][2 * (l & 1) + 1] ^ 0x80808080u, w + 2);
-      m = __builtin_bit_cast(f16, f.d[h]);
+      m = __builtin_bit_cast(f16, pair_at(f.d, h));
     } else {
       const int k = 2 * (l & 1);  // byte i's low nibble is weight i, its high nibble weight 16 + i
       const uint32_t q0 = f.qs[h][k] >> (4 * (l >> 1)), q1 = f.qs[h][k + 1] >> (4 * (l >> 1));
@@ -260,7 +263,7 @@ __device__ __forceinline__ void decode_linear4(const RunPair<KIND>& f, int h, in
         const uint32_t ls = ((f.sl >> (8 * g + 4 * h)) & 15) | (((f.dh >> (16 + 2 * ib)) & 3) << 4);
         m = (f16)(int16_t)((int)ls - 32);
       } else {
-        m = __builtin_bit_cast(f16, f.d[h]);
+        m = __builtin_bit_cast(f16, pair_at(f.d, h));
       }
     }
     fold_pairs<SPLIT>(w, h2v{m, m}, lo);
@@ -708,25 +711,23 @@ __device__ __forceinline__ void dword_fields(const uint8_t* lds, uint32_t off, i
     uint32_t w[17];
 #pragma unroll
     for (int k = 0; k < 17; ++k) w[k] = lds_at<uint32_t>(lds, off + 68 * g + 4 * k);
+    auto at2 = [&](int k) { return __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2); };
     f.d[0] = (uint16_t)(w[0] & 0xffffu);
     f.d[1] = (uint16_t)(w[8] >> 16);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      f.q[k / 4][k % 4] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
-      f.q[2 + k / 4][k % 4] = w[9 + k];
-    }
+    f.q[0] = u32x4{at2(0), at2(1), at2(2), at2(3)};
+    f.q[1] = u32x4{at2(4), at2(5), at2(6), at2(7)};
+    f.q[2] = u32x4{w[9], w[10], w[11], w[12]};
+    f.q[3] = u32x4{w[13], w[14], w[15], w[16]};
   } else {
     static_assert(KIND == K_IQ4_NL || KIND == K_Q4_0, "the dword types");  // 36 bytes: d, 16 code bytes, twice
     uint32_t w[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) w[k] = lds_at<uint32_t>(lds, off + 36 * g + 4 * k);
+    auto at2 = [&](int k) { return __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2); };
     f.d[0] = (uint16_t)(w[0] & 0xffffu);
     f.d[1] = (uint16_t)(w[4] >> 16);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      f.qs[0][k] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
-      f.qs[1][k] = w[5 + k];
-    }
+    f.qs[0] = u32x4{at2(0), at2(1), at2(2), at2(3)};
+    f.qs[1] = u32x4{w[5], w[6], w[7], w[8]};
   }
 }
 // The first byte of a dword type's slot at step k: the step's dword, or (a partial last step) as many dwords before

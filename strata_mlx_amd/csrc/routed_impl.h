@@ -311,6 +311,38 @@ struct GluParams {
 __device__ __forceinline__ int glu_x_slot(int j, int i) { return 8 * j + (i ^ (j & 7)); }
 __device__ __forceinline__ int x_piece_slot(int c) { return glu_x_slot(c >> 3, c & 7); }
 
+// bfloat16 tokens on their way to LDS: the largest magnitude of a wave's 16-byte pieces (bfloat16 bits), a token's
+// exponent from its waves' (row_exponent), and a piece divided by that power of two as float16 (exact for every value
+// within 2^31 of the token's largest).
+__device__ __forceinline__ uint32_t bf16_pieces_max(const u32x4& v) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 m = us2{0, 0};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, v[i] & 0x7fff7fffu));
+  uint32_t u = max((uint32_t)m[0], (uint32_t)m[1]);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) u = max(u, (uint32_t)__shfl_xor((int)u, d));
+  return u;
+}
+__device__ __forceinline__ int token_exponent(const uint32_t* waves_max, int waves) {
+  uint32_t u = 0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w)
+    if (w < waves) u = max(u, waves_max[w]);
+  return row_exponent(u << 16);
+}
+__device__ __forceinline__ u32x4 bf16_piece_scaled(const u32x4& v, int ex) {
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float lo = __builtin_ldexpf(__uint_as_float(v[i] << 16), -ex);
+    const float hi = __builtin_ldexpf(__uint_as_float(v[i] & 0xffff0000u), -ex);
+    o[i] = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<f16>(lo)) |
+           ((uint32_t)__builtin_bit_cast(uint16_t, from_f32<f16>(hi)) << 16);
+  }
+  return o;
+}
+
 // The unit's two rows decoded and multiplied (gate and up, or rows 2 i and 2 i + 1), and their sums met over the
 // wave: the first row's total and the second's, the same in every lane (read into scalars).
 template <int KIND, bool TWO = false>
@@ -341,13 +373,20 @@ __device__ __forceinline__ void glu_unit(typename Routed<KIND>::Fields (&f)[2], 
 // ROUTE (one token, 256 experts at most): the pairs' experts are chosen in the launch from the router's logits, by
 // wave 0 of every workgroup while the table and the token go to LDS (the same choice as top_k's); workgroup 0 writes
 // it out for the down and combine launches. It spares the router's launch the count and the choice at its end.
-template <int KIND, int UPW, int MODE, bool SHARED = false, bool ROUTE = false>
+//
+// XT bfloat16 (GLU1, GLUN): each token is scaled by a power of two into float16's upper range on its way to LDS (its
+// largest magnitude found over the waves that hold it: one more barrier), the sums are scaled back, and g, u and h are
+// rounded to bfloat16.
+template <int KIND, int UPW, int MODE, bool SHARED = false, bool ROUTE = false, typename XT = f16>
 __global__ __launch_bounds__((glu_threads<KIND, MODE>()), (glu_threads<KIND, MODE>() / 256)) void routed_glu_kernel(
     GluParams p) {
   constexpr int kGluThreads = glu_threads<KIND, MODE>(), kGluWaves = kGluThreads / 64;
   typedef Routed<KIND> R;
   typedef typename R::Fields Fields;
   constexpr bool kOne = MODE == ONE || MODE == ONE32;
+  constexpr bool kBf16 = std::is_same<XT, bf16_t>::value;
+  static_assert(!kBf16 || (!kOne && !SHARED && !ROUTE && kGluThreads == 1024), "bfloat16 tokens: gate and up");
+  __shared__ uint32_t token_max[kBf16 ? kGluMaxTokens : 1][8];  // by the waves that hold a token's pieces
   // units whose rows are in registers at once: ONE32 holds two parts of the token, SHARED the shared expert's unit
   constexpr int kMaxBuffers = MODE == ONE32 ? 1 : SHARED ? R::kBuffers - 1 : R::kBuffers;
   constexpr int kBuffers = UPW < kMaxBuffers ? UPW : kMaxBuffers;  // units whose rows are in registers at once
@@ -485,6 +524,18 @@ __global__ __launch_bounds__((glu_threads<KIND, MODE>()), (glu_threads<KIND, MOD
       *l2 = u32x2{lo[0], lo[1]};
     }
   } else {
+    if constexpr (kBf16) {  // a wave's pieces of one load are one token's
+#pragma unroll
+      for (int k = 0; k < kPieceLoads; ++k) {
+        const uint32_t u = bf16_pieces_max(xpiece[k]);
+        const int c = tid + k * kGluThreads;
+        if (lane == 0 && c < 512 * p.tokens) token_max[c >> 9][(c >> 6) & 7] = u;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kPieceLoads; ++k)
+        xpiece[k] = bf16_piece_scaled(xpiece[k], token_exponent(token_max[min(tid + k * kGluThreads, 512 * p.tokens - 1) >> 9], 8));
+    }
 #pragma unroll
     for (int k = 0; k < kPieceLoads; ++k) {
       const int c = min(tid + k * kGluThreads, 512 * p.tokens - 1);  // threads past the pieces write one again
@@ -601,15 +652,20 @@ __global__ __launch_bounds__((glu_threads<KIND, MODE>()), (glu_threads<KIND, MOD
       if (w_row + 1 < p.rows) p.out_gate[w_row + 1] = from_f32<f16>(uv);
     } else {
       const int64_t o = (int64_t)w_pair * p.rows + w_row;
-      f16 gq = from_f32<f16>(gv), uq = from_f32<f16>(uv), hq;
-      if (w_bad) {
-        gq = uq = hq = (f16)__builtin_nanf("");
-      } else {
-        hq = from_f32<f16>(swiglu_rounded<f16>(gq, uq));
+      if constexpr (kBf16) {
+        const int te = token_exponent(token_max[w_pair / p.share], 8);
+        gv = __builtin_ldexpf(gv, te);
+        uv = __builtin_ldexpf(uv, te);
       }
-      if (p.out_gate != nullptr) p.out_gate[o] = gq;
-      if (p.out_up != nullptr) p.out_up[o] = uq;
-      p.h[o] = hq;
+      XT gq = from_f32<XT>(gv), uq = from_f32<XT>(uv), hq;
+      if (w_bad) {
+        gq = uq = hq = from_f32<XT>(__builtin_nanf(""));
+      } else {
+        hq = from_f32<XT>(swiglu_rounded<XT>(gq, uq));
+      }
+      if (p.out_gate != nullptr) reinterpret_cast<XT*>(p.out_gate)[o] = gq;
+      if (p.out_up != nullptr) reinterpret_cast<XT*>(p.out_up)[o] = uq;
+      reinterpret_cast<XT*>(p.h)[o] = hq;
     }
   }
   if constexpr (SHARED) {
@@ -659,8 +715,11 @@ struct DownParams {
 // its shared rows' fields through the routed decode and spilled 60 registers). At eight pairs of 4096 rows the
 // 256 workgroups take 4096 shared rows: the routed launch alone 8.4 us a layer, with the shared down 8.7-9.1 us,
 // the two launches apart 13.2 us.
-template <int KIND, int S, int UPW, bool SHARED = false>
+template <int KIND, int S, int UPW, bool SHARED = false, typename XT = f16>
 __global__ __launch_bounds__(kGluThreads, 4) void routed_down_kernel(DownParams p) {
+  constexpr bool kBf16 = std::is_same<XT, bf16_t>::value;  // the token scaled into float16 (routed_glu_kernel)
+  static_assert(!kBf16 || !SHARED, "the shared form: float16");
+  __shared__ uint32_t token_max[8];
   typedef Routed<KIND> R;
   typedef Routed<K_Q4_K> RS;
   constexpr int kPairs = 8 * S;        // run pairs of a row
@@ -675,13 +734,22 @@ __global__ __launch_bounds__(kGluThreads, 4) void routed_down_kernel(DownParams 
 
   // the table entry this thread expands and a piece of the pair's token (and of the shared expert's), asked for first
   const uint64_t entry = R::fetch(tid);
-  const u32x4 xpiece = reinterpret_cast<const u32x4*>(p.x + (int64_t)(pair / p.share) * (8 * kPieces))[tid % kPieces];
+  u32x4 xpiece = reinterpret_cast<const u32x4*>(p.x + (int64_t)(pair / p.share) * (8 * kPieces))[tid % kPieces];
   u32x4 spiece;
   if constexpr (SHARED) spiece = reinterpret_cast<const u32x4*>(p.s_x)[tid % kPieces];
   const uint32_t e = p.idx[pair];
   const bool bad = e >= p.experts;
   const uint8_t* mat = p.blocks + (int64_t)(bad ? 0u : e) * p.mat_bytes;
   R::fill(tab, tid, entry);
+  int ex = 0;
+  if constexpr (kBf16) {  // the first kPieces threads' waves hold every piece
+    static_assert(kPieces % 64 == 0 && kPieces <= 512, "whole waves");
+    const uint32_t u = bf16_pieces_max(xpiece);
+    if (lane == 0 && tid < kPieces) token_max[wave] = u;
+    __syncthreads();
+    ex = token_exponent(token_max, kPieces / 64);
+    xpiece = bf16_piece_scaled(xpiece, ex);
+  }
   {
     const int c = tid % kPieces;  // threads past the token's pieces write the same bytes again
     xs[glu_x_slot(c >> 3, c & 7)] = xpiece;
@@ -730,7 +798,8 @@ __global__ __launch_bounds__(kGluThreads, 4) void routed_down_kernel(DownParams 
       acc += lanes_apart(acc, 4);
       const int r = r0[k] + sub;
       if (m == 0 && r < p.rows)
-        p.out[(int64_t)pair * p.rows + r] = bad ? (f16)__builtin_nanf("") : from_f32<f16>(acc);
+        reinterpret_cast<XT*>(p.out)[(int64_t)pair * p.rows + r] =
+            from_f32<XT>(bad ? __builtin_nanf("") : kBf16 ? __builtin_ldexpf(acc, ex) : acc);
     }
   };
 
@@ -790,19 +859,19 @@ bool routed_down_takes(const MatvecParams& p) {
          p.glu_out == nullptr && p.experts <= INT32_MAX && p.pairs <= 65535;
 }
 
-template <int KIND, int S, int UPW, bool SHARED = false>
+template <int KIND, int S, int UPW, bool SHARED = false, typename XT = f16>
 int launch_down_su(DownParams& p, int units_per_pair, hipStream_t s) {
   const int per_group = kGluWaves * UPW;
   p.groups_per_pair = (units_per_pair + per_group - 1) / per_group;
   const int64_t groups = (int64_t)p.groups_per_pair * p.pairs;
   if (groups > INT32_MAX) return STRATA_ERR_SHAPE;
   if (SHARED && (p.s_rows + 7) / 8 > 2 * groups) return STRATA_ERR_SHAPE;  // two shared units a workgroup
-  hipLaunchKernelGGL((routed_down_kernel<KIND, S, UPW, SHARED>), dim3((unsigned)groups), dim3(kGluThreads), 0, s, p);
+  hipLaunchKernelGGL((routed_down_kernel<KIND, S, UPW, SHARED, XT>), dim3((unsigned)groups), dim3(kGluThreads), 0, s, p);
   STRATA_CHECK_LAUNCH();
   return STRATA_OK;
 }
 
-template <int KIND>
+template <int KIND, typename XT = f16>
 int launch_routed_down(const MatvecParams& mp, hipStream_t s) {
   if constexpr (!routed_kind(KIND)) {
     return STRATA_ERR_SHAPE;
@@ -833,12 +902,14 @@ int launch_routed_down(const MatvecParams& mp, hipStream_t s) {
       p.s_out = reinterpret_cast<f16*>(mp.shared_out);
       p.s_rows = mp.shared_rows;
       p.s_row_bytes = mp.shared_row_bytes;
-      if (mp.cols != 1536 || two) return STRATA_ERR_SHAPE;
+      if (mp.cols != 1536 || two || !std::is_same<XT, f16>::value) return STRATA_ERR_SHAPE;
       return launch_down_su<KIND, 3, 1, true>(p, units_per_pair, s);
     }
     if (mp.cols == 1536)
-      return two ? launch_down_su<KIND, 3, 2>(p, units_per_pair, s) : launch_down_su<KIND, 3, 1>(p, units_per_pair, s);
-    return two ? launch_down_su<KIND, 5, 2>(p, units_per_pair, s) : launch_down_su<KIND, 5, 1>(p, units_per_pair, s);
+      return two ? launch_down_su<KIND, 3, 2, false, XT>(p, units_per_pair, s)
+                 : launch_down_su<KIND, 3, 1, false, XT>(p, units_per_pair, s);
+    return two ? launch_down_su<KIND, 5, 2, false, XT>(p, units_per_pair, s)
+               : launch_down_su<KIND, 5, 1, false, XT>(p, units_per_pair, s);
   }
 }
 
@@ -864,23 +935,23 @@ bool routed_one_takes(const MatvecParams& p) {
          p.rows <= INT32_MAX / 2;
 }
 
-template <int KIND, int MODE, bool SHARED = false>
+template <int KIND, int MODE, bool SHARED = false, typename XT = f16>
 int launch_glu_upw(GluParams& p, int upw, dim3 grid, hipStream_t s) {
   const dim3 block(glu_threads<KIND, MODE>());
   switch (upw) {
-    case 1: hipLaunchKernelGGL((routed_glu_kernel<KIND, 1, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 2: hipLaunchKernelGGL((routed_glu_kernel<KIND, 2, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 3: hipLaunchKernelGGL((routed_glu_kernel<KIND, 3, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 4: hipLaunchKernelGGL((routed_glu_kernel<KIND, 4, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 6: hipLaunchKernelGGL((routed_glu_kernel<KIND, 6, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 8: hipLaunchKernelGGL((routed_glu_kernel<KIND, 8, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 12: hipLaunchKernelGGL((routed_glu_kernel<KIND, 12, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 15: hipLaunchKernelGGL((routed_glu_kernel<KIND, 15, MODE, SHARED>), grid, block, 0, s, p); break;
-    case 16: hipLaunchKernelGGL((routed_glu_kernel<KIND, 16, MODE, SHARED>), grid, block, 0, s, p); break;
+    case 1: hipLaunchKernelGGL((routed_glu_kernel<KIND, 1, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 2: hipLaunchKernelGGL((routed_glu_kernel<KIND, 2, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 3: hipLaunchKernelGGL((routed_glu_kernel<KIND, 3, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 4: hipLaunchKernelGGL((routed_glu_kernel<KIND, 4, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 6: hipLaunchKernelGGL((routed_glu_kernel<KIND, 6, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 8: hipLaunchKernelGGL((routed_glu_kernel<KIND, 8, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 12: hipLaunchKernelGGL((routed_glu_kernel<KIND, 12, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 15: hipLaunchKernelGGL((routed_glu_kernel<KIND, 15, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
+    case 16: hipLaunchKernelGGL((routed_glu_kernel<KIND, 16, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
     case 20:
-      if constexpr (MODE == ONE) hipLaunchKernelGGL((routed_glu_kernel<KIND, 20, MODE, SHARED>), grid, block, 0, s, p);
+      if constexpr (MODE == ONE) hipLaunchKernelGGL((routed_glu_kernel<KIND, 20, MODE, SHARED, false, XT>), grid, block, 0, s, p);
       break;
-    default: hipLaunchKernelGGL((routed_glu_kernel<KIND, 24, MODE, SHARED>), grid, block, 0, s, p); break;
+    default: hipLaunchKernelGGL((routed_glu_kernel<KIND, 24, MODE, SHARED, false, XT>), grid, block, 0, s, p); break;
   }
   STRATA_CHECK_LAUNCH();
   return STRATA_OK;
@@ -903,7 +974,7 @@ int glu_units_a_wave(int64_t units) {
   return KIND == K_IQ3_S ? 16 : 24;
 }
 
-template <int KIND, int MODE, bool SHARED = false>
+template <int KIND, int MODE, bool SHARED = false, typename XT = f16>
 int launch_glu_mode(GluParams& p, hipStream_t s) {
   const int64_t units = (int64_t)p.na * p.nb;
   const int upw = glu_units_a_wave<KIND, MODE>(units);
@@ -915,7 +986,7 @@ int launch_glu_mode(GluParams& p, hipStream_t s) {
   p.wave_b = p.waves % p.nb;
   // one shared unit a wave at most; above 12 units a wave the shared unit's rows spill registers
   if (SHARED && (p.s_rows > p.waves || upw > 12)) return STRATA_ERR_SHAPE;
-  return launch_glu_upw<KIND, MODE, SHARED>(p, upw, dim3((unsigned)(waves / kWaves)), s);
+  return launch_glu_upw<KIND, MODE, SHARED, XT>(p, upw, dim3((unsigned)(waves / kWaves)), s);
 }
 
 // The ROUTE form: the one-token shared form at three units a wave (eight pairs of 1536 rows), the choice of experts
@@ -938,7 +1009,7 @@ int launch_glu_route(GluParams& p, hipStream_t s) {
   return STRATA_OK;
 }
 
-template <int KIND>
+template <int KIND, typename XT = f16>
 int launch_routed_glu(const MatvecParams& mp, hipStream_t s) {
   if constexpr (!routed_kind(KIND)) {
     return STRATA_ERR_SHAPE;
@@ -959,6 +1030,7 @@ int launch_routed_glu(const MatvecParams& mp, hipStream_t s) {
     p.share = mp.share;
     p.tokens = mp.pairs / mp.share;
     if (mp.shared[0] != nullptr) {  // the shared expert's gate and up in the same launch: one token
+      if (!std::is_same<XT, f16>::value) return STRATA_ERR_SHAPE;
       if (p.tokens != 1 || mp.shared_rows < 1) return STRATA_ERR_SHAPE;
       if (mp.route_logits != nullptr) {  // and the choice of experts
         p.r_logits = mp.route_logits;
@@ -983,11 +1055,11 @@ int launch_routed_glu(const MatvecParams& mp, hipStream_t s) {
     if (p.tokens > 1) {
       p.na = p.pairs;
       p.nb = p.rows;
-      return launch_glu_mode<KIND, GLUN>(p, s);
+      return launch_glu_mode<KIND, GLUN, false, XT>(p, s);
     }
     p.na = p.pairs;
     p.nb = p.rows;
-    return launch_glu_mode<KIND, GLU1>(p, s);
+    return launch_glu_mode<KIND, GLU1, false, XT>(p, s);
   }
 }
 

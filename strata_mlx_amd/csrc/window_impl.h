@@ -85,6 +85,104 @@ __device__ __forceinline__ f16x8 own_mins(const RunPair<KIND>& f, int g) {
   return __builtin_bit_cast(f16x8, u32x4{mn[0], mn[1], 0u, 0u});
 }
 
+// The tokens of a workgroup's slots into float16's upper range, each by a power of two (exact down to 2^-31 of its
+// largest), in the registers of the waves that hold them: a slot's largest magnitude over its lanes and waves (peak).
+// ex_out: the exponents of the slots that the lane writes; sums: the lane's run sums (the types with mins).
+template <int KIND, typename XT, int SPW>
+__device__ __forceinline__ void scale_tokens(u32x4 (&a)[SPW][2][4], uint32_t (&sums)[SPW][2], int (&ex_out)[4],
+                                             uint32_t (*peak)[kSlots], int wave, int waves, int n, int g) {
+  us2 m = us2{0, 0};  // magnitudes compare as their bits do
+#pragma unroll
+  for (int s = 0; s < SPW; ++s)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, a[s][h][q][c] & 0x7fff7fffu));
+  uint32_t u = max((uint32_t)m[0], (uint32_t)m[1]);
+  u = max(u, (uint32_t)__shfl_xor((int)u, 16));
+  u = max(u, (uint32_t)__shfl_xor((int)u, 32));
+  if (g == 0) peak[wave][n] = u;
+  __syncthreads();
+  auto exponent = [&](int slot) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int w = 0; w < kMaxWaves; ++w) v = max(v, w < waves ? peak[w][slot] : 0u);
+    return row_exponent(__float_as_uint(to_f32(__builtin_bit_cast(XT, (uint16_t)v))));
+  };
+  const int ex = exponent(n);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ex_out[j] = exponent(4 * g + j);
+  // float16 tokens by three powers of two (2^38 at most together, 2^15 each), each product exact
+  const int e1 = min(-ex, 15), e2 = min(-ex - e1, 15), e3 = -ex - e1 - e2;
+  const f16 b1 = (f16)__builtin_ldexpf(1.0f, e1), b2 = (f16)__builtin_ldexpf(1.0f, e2), b3 = (f16)__builtin_ldexpf(1.0f, e3);
+#pragma unroll
+  for (int s = 0; s < SPW; ++s) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t v = a[s][h][q][c];
+          uint32_t w;
+          if constexpr (std::is_same<XT, bf16_t>::value) {  // exact down to 2^-31 of the token's largest
+            w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(
+                                                 __builtin_ldexpf(__uint_as_float(v << 16), -ex),
+                                                 __builtin_ldexpf(__uint_as_float(v & 0xffff0000u), -ex)));
+          } else {
+            w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, v) * h2v{b1, b1} * h2v{b2, b2} * h2v{b3, b3});
+          }
+          a[s][h][q][c] = w;
+          if constexpr (kHasMin<KIND>)
+            sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(strata_mv::h2_t, w),
+                                         __builtin_bit_cast(strata_mv::h2_t, 0x3C003C00u), sum, false);
+        }
+      if constexpr (kHasMin<KIND>) sums[s][h] = split_sum(sum);
+    }
+  }
+}
+
+// One K step's products added to acc: the step's fields against the lane's operands of it.
+template <int KIND>
+__device__ __forceinline__ void add_step(const RunPair<KIND>& f, const u32x4 (&a)[2][4], const uint32_t (&sums)[2], int g,
+                                         const DirectTables<KIND>& tab, f32x4& acc) {
+  f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto run = [&](auto hc) {  // run h a constant from the start: the fields' pairs indexed by it stay in registers
+    constexpr int h = decltype(hc)::value;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t w[4], lo[4];
+      if constexpr (strata_prompt::kInexact<KIND>)
+        strata_prompt::decode_linear4<KIND, true>(f, h, g, q, w, lo, tab);
+      else
+        strata_prompt::decode_folded4<KIND>(f, h, g, q, w, tab);
+      part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[h][q]),
+                                                    __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[2], w[3]}), part, 0, 0, 0);
+      if constexpr (strata_prompt::kInexact<KIND>)
+        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[h][q]),
+                                                      __builtin_bit_cast(f16x8, u32x4{lo[0], lo[1], lo[2], lo[3]}), part,
+                                                      0, 0, 0);
+    }
+  };
+  run(std::integral_constant<int, 0>());
+  run(std::integral_constant<int, 1>());
+  const float d = strata_prompt::step_scale<KIND>(f);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(d, part[j], acc[j]);
+  if constexpr (kHasMin<KIND>) {
+    const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4 mm = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+        __builtin_bit_cast(f16x8, u32x4{sums[0], sums[1], 0u, 0u}), own_mins<KIND>(f, g), z, 0, 0, 0);
+    const float dm = strata_prompt::kSumScale * strata_mv::half_bits(f.dd >> 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(-dm, mm[j], acc[j]);
+  }
+}
+
 template <int KIND>
 constexpr bool kStagedRows = KIND == K_Q4_K || KIND == K_Q6_K || KIND == K_Q8_0;
 // 16-byte pieces of a wave's part of a row, from the aligned one that holds its first byte (an even one), and the pitch
@@ -165,7 +263,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
   const uint32_t slab0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)slabs + (uint32_t)(wave * 2 * kSlab));
   auto stage = [&](int i, int which) {
     if constexpr (STAGED) {
-      i = min(i, groups - 1);
+      if (i >= groups) return;  // nothing to ask for past the last group
       const uint8_t* base = p.blocks + (int64_t)i * 16 * p.row_bytes;
       if (16 * i + 16 > p.rows) {  // the last group, cut short: rows past the matrix read its last
 #pragma unroll
@@ -236,58 +334,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
   uint32_t sums[SPW][2];
   int ex_out[4] = {0, 0, 0, 0};  // the exponents of the slots the lane writes
   if constexpr (kScaled) {
-    us2 m = us2{0, 0};  // magnitudes compare as their bits do
-#pragma unroll
-    for (int s = 0; s < SPW; ++s)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, a[s][h][q][c] & 0x7fff7fffu));
-    uint32_t u = max((uint32_t)m[0], (uint32_t)m[1]);
-    u = max(u, (uint32_t)__shfl_xor((int)u, 16));
-    u = max(u, (uint32_t)__shfl_xor((int)u, 32));
-    if (g == 0) peak[wave][n] = u;
-    __syncthreads();
-    auto exponent = [&](int slot) {
-      uint32_t v = 0;
-#pragma unroll
-      for (int w = 0; w < kMaxWaves; ++w) v = max(v, w < waves ? peak[w][slot] : 0u);
-      return row_exponent(__float_as_uint(to_f32(__builtin_bit_cast(XT, (uint16_t)v))));
-    };
-    const int ex = exponent(n);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) ex_out[j] = exponent(4 * g + j);
-    // float16 tokens by two powers of two (up to 2^39 together), each product exact
-    const f16 by = (f16)__builtin_ldexpf(1.0f, -ex / 2), by2 = (f16)__builtin_ldexpf(1.0f, -ex - -ex / 2);
-#pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const uint32_t v = a[s][h][q][c];
-            uint32_t w;
-            if constexpr (std::is_same<XT, bf16_t>::value) {  // exact down to 2^-31 of the token's largest
-              w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(
-                                                   __builtin_ldexpf(__uint_as_float(v << 16), -ex),
-                                                   __builtin_ldexpf(__uint_as_float(v & 0xffff0000u), -ex)));
-            } else {
-              w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, v) * h2v{by, by} * h2v{by2, by2});
-            }
-            a[s][h][q][c] = w;
-            if constexpr (kHasMin<KIND>)
-              sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(strata_mv::h2_t, w),
-                                           __builtin_bit_cast(strata_mv::h2_t, 0x3C003C00u), sum, false);
-          }
-        if constexpr (kHasMin<KIND>) sums[s][h] = split_sum(sum);
-      }
-    }
+    scale_tokens<KIND, XT, SPW>(a, sums, ex_out, peak, wave, waves, n, g);
   }
   __syncthreads();  // the tables
 
@@ -296,7 +343,10 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
     RunPair<KIND> fn[STAGED ? 1 : SPW];
     if constexpr (STAGED) {  // this group's loads are in (the next one's may be in flight); its fields, then the slab
       constexpr int kNext = kLoads;
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNext) : "memory");
+      if (next < groups)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNext) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const uint8_t* slot = slabs + (wave * 2 + (it & 1)) * kSlab + 16 * kPitch<KIND, SPW> * n;
 #pragma unroll
       for (int s = 0; s < SPW; ++s) staged_fields<KIND>(slot, at[s], g, f[s]);
@@ -307,37 +357,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
     }
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-      f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          uint32_t w[4], lo[4];
-          if constexpr (strata_prompt::kInexact<KIND>)
-            strata_prompt::decode_linear4<KIND, true>(f[s], h, g, q, w, lo, tab);
-          else
-            strata_prompt::decode_folded4<KIND>(f[s], h, g, q, w, tab);
-          part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[s][h][q]),
-                                                        __builtin_bit_cast(f16x8, u32x4{w[0], w[1], w[2], w[3]}), part,
-                                                        0, 0, 0);
-          if constexpr (strata_prompt::kInexact<KIND>)
-            part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[s][h][q]),
-                                                          __builtin_bit_cast(f16x8, u32x4{lo[0], lo[1], lo[2], lo[3]}),
-                                                          part, 0, 0, 0);
-        }
-      const float d = strata_prompt::step_scale<KIND>(f[s]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(d, part[j], acc[j]);
-      if constexpr (kHasMin<KIND>) {
-        const f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
-        const f32x4 mm = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(f16x8, u32x4{sums[s][0], sums[s][1], 0u, 0u}), own_mins<KIND>(f[s], g), z, 0, 0, 0);
-        const float dm = strata_prompt::kSumScale * strata_mv::half_bits(f[s].dd >> 16);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(-dm, mm[j], acc[j]);
-      }
-    }
+    for (int s = 0; s < SPW; ++s) add_step<KIND>(f[s], a[s], sums[s], g, tab, acc);
     f32x4(*buf)[64] = red[it & 1];
     buf[wave][lane] = acc;
     strata_prompt::lds_barrier();  // waits for LDS only: the next group's fields stay in flight
@@ -369,14 +389,17 @@ __global__ __launch_bounds__(64 * kMaxWaves, 2) void window_kernel(WindowParams 
     }
     i = next;
   }
-  if constexpr (STAGED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the rows asked for past the last
 }
+
+constexpr int kMinRows = 512;  // (float16) rows below which the matvecs keep a window
 
 // Whether window_kernel takes a dense product: up to 16 tokens whose rows lie at 16-byte boundaries, rows of whole
 // run pairs (whole steps in the types with blocks of 256) and at most 4096 inputs; listed rows where the matrix's
 // byte offsets fit 32 bits.
-inline bool window_takes(int kind, const WindowParams& p) {
-  return strata_prompt::tiles_take(kind, p.cols) && p.cols <= kMaxCols && p.tokens >= 1 && p.tokens <= kSlots &&
+// A float16 layer of fewer than 512 rows, at most 32 row groups, stays on the matvecs, which spread it over more CUs (two
+// tokens of Q8_0 64 x 2048 5.8 against 6.0 us) and give a token the bits it has alone.
+inline bool window_takes(int kind, const WindowParams& p, bool f16_tokens) {
+  return (!f16_tokens || p.src_rows >= kMinRows) && strata_prompt::tiles_take(kind, p.cols) && p.cols <= kMaxCols && p.tokens >= 1 && p.tokens <= kSlots &&
          ((uintptr_t)p.x & 15) == 0 &&
          (p.ids == nullptr || (int64_t)p.src_rows * p.row_bytes < ((int64_t)1 << 32));
 }

@@ -41,14 +41,14 @@ def check(gpu, kind, rows, cols, tokens, dtype, spread=0):
 
 
 @pytest.mark.parametrize("kind", K_TYPES)
-@pytest.mark.parametrize("rows, cols, tokens", [(100, 256, 2), (16, 1536, 5), (1000, 2560, 8), (4100, 4096, 16)])
+@pytest.mark.parametrize("rows, cols, tokens", [(600, 256, 2), (16, 1536, 5), (1000, 2560, 8), (4100, 4096, 16)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_types_of_256_weight_blocks(gpu, kind, rows, cols, tokens, dtype):
     check(gpu, kind, rows, cols, tokens, dtype)
 
 
 @pytest.mark.parametrize("kind", SMALL)
-@pytest.mark.parametrize("rows, cols, tokens", [(33, 64, 3), (40, 640, 16), (1000, 2240, 5), (4100, 4096, 7)])
+@pytest.mark.parametrize("rows, cols, tokens", [(33, 64, 3), (520, 640, 16), (1000, 2240, 5), (4100, 4096, 7)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_types_of_smaller_blocks(gpu, kind, rows, cols, tokens, dtype):
     check(gpu, kind, rows, cols, tokens, dtype)
