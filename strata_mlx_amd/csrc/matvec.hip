@@ -94,8 +94,23 @@ bool rwin_wanted(int kind, const MatvecParams& p, int dtype, bool with_h) {
   return !(routed && (p.cols == 1536 || p.cols == 2560) && p.pairs <= kRoutedPairs);
 }
 
-constexpr int64_t kShortRows = 8192;
-constexpr int64_t kLongRows = 16384;  // above, one float16 token of Q8_0 takes the window kernel
+// Tokens from which a dense product goes to window_kernel. bfloat16: one, its matvec being the generic one (Q6_K
+// 4096 x 4096 17.8 -> 11.5 us). float16: two, but for
+//   one token of a long Q8_0 layer (151936 x 4096 161 -> 109 us; at 12288 rows and below the one-token kernels are as fast);
+//   short layers of long rows, whose launch is mostly its prologue: 2048 x 4096 Q6_K at two tokens 6.7 us on the matvec
+//   against 7.1, at three 8.1 against 7.2; the types with mins (scaled tokens) and Q3_K (rows not staged) up to 4096
+//   rows: Q4_K 1024 x 4096 at three 7.9 against 8.8, at four 9.4 against 9.1; Q3_K 8.8 against 9.9, 10.6 against 10.2;
+//   layers of the types with mins up to 8192 rows (Q4_K 4096 x 4096 at two 7.8 against 9.5, 12288 rows 16.1 against
+//   14.3) and IQ3_S (4096 x 4096 at two 7.0 against 7.7, at three 10.1 against 7.9).
+int window_from(int kind, int64_t rows, int64_t cols, int dtype) {
+  if (dtype == DT_BF16 || (kind == K_Q8_0 && rows > 16384)) return 1;
+  const bool mins = kind == K_Q4_K || kind == K_Q5_K;
+  if (cols > 2560) {
+    if ((mins || kind == K_Q3_K) && rows <= 4096) return 4;
+    if (rows <= 2048) return 3;
+  }
+  return (mins && rows <= 8192) || kind == K_IQ3_S ? 3 : 2;
+}
 
 int window_by_kind(int kind, const strata_window::WindowParams& p, int dtype, hipStream_t s) {
   switch (kind) {
@@ -462,14 +477,8 @@ int strata_dense_matvec(int kind, const void* blocks, int64_t rows, int64_t cols
   p.cols = (int)cols;
   p.tokens = (int)tokens;
   p.mode = MODE_DENSE;
-  // 16-bit windows of two tokens or more on MFMA, the rows decoded once for all of them. One bfloat16 token too, whose
-  // matvec is the generic one (Q6_K 4096 x 4096 17.8 -> 10.9 us), and one float16 token of a long Q8_0 matrix
-  // (151936 x 4096 161 -> 109 us; at 12288 rows and below the one-token kernels are as fast).
-  const bool one = x_dtype == DT_BF16 || (kind == K_Q8_0 && rows > kLongRows);
-  // Two float16 tokens of a short Q4_K or Q5_K layer stay on the matvec, which scales no tokens (4096 x 4096 7.8
-  // against 9.5 us, 12288 rows 16.1 against 14.3).
-  const bool three = x_dtype == DT_F16 && (kind == K_Q4_K || kind == K_Q5_K) && rows <= kShortRows;
-  if (x_dtype == out_dtype && x_dtype != DT_F32 && tokens >= (one ? 1 : three ? 3 : 2)) {
+  // 16-bit windows on MFMA, the rows decoded once for all tokens, from as many tokens as it pays at
+  if (x_dtype == out_dtype && x_dtype != DT_F32 && tokens >= window_from(kind, rows, cols, x_dtype)) {
     strata_window::WindowParams w = {};
     w.blocks = p.blocks[0];
     w.x = x;

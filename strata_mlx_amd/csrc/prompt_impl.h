@@ -590,13 +590,14 @@ __device__ __forceinline__ void run_chunk(const PromptParams& p, const DirectTab
 // on a CU; at two (a third row buffer, or the IQ3_XXS codebook with its signs folded in, 32 KB) or at four (128
 // registers, spilled) the kernel ran slower.
 //
-// Q4_K, Q5_K, Q6_K, IQ4_NL, Q4_0 and Q8_0 rows too (kDwordRows): loaded straight into registers, the 16-byte loads of
+// Q4_K, Q5_K, Q6_K, IQ4_NL, Q4_0, Q5_0 and Q8_0 rows too (kDwordRows): loaded straight into registers, the 16-byte loads of
 // those whose fields lie 2 or 4 bytes past a boundary ran several times longer still. Their slots are an odd number of
 // dwords apart, so that reads of one dword spread over the banks, and each field is put together from dwords. Down of
 // a layer of 256 Q6_K experts at 384 tokens 684 -> 402 us (33 spilled registers less at two waves a SIMD among it),
 // gate and up in Q4_K 764 -> 600.
 template <int KIND>
-constexpr bool kDwordRows = KIND == K_Q4_K || KIND == K_Q5_K || KIND == K_Q6_K || KIND == K_IQ4_NL || KIND == K_Q4_0 || KIND == K_Q8_0;
+constexpr bool kDwordRows = KIND == K_Q4_K || KIND == K_Q5_K || KIND == K_Q6_K || KIND == K_IQ4_NL || KIND == K_Q4_0 ||
+                            KIND == K_Q5_0 || KIND == K_Q8_0;
 template <int KIND>
 constexpr bool kStagedKind = KIND == K_IQ3_S || KIND == K_IQ3_XXS || KIND == K_Q2_0 || kDwordRows<KIND>;
 template <int KIND>
@@ -718,6 +719,17 @@ __device__ __forceinline__ void dword_fields(const uint8_t* lds, uint32_t off, i
     f.q[1] = u32x4{at2(4), at2(5), at2(6), at2(7)};
     f.q[2] = u32x4{w[9], w[10], w[11], w[12]};
     f.q[3] = u32x4{w[13], w[14], w[15], w[16]};
+  } else if constexpr (KIND == K_Q5_0) {  // 44 bytes: d, 4 high-bit bytes, 16 code bytes, twice
+    uint32_t w[11];
+#pragma unroll
+    for (int k = 0; k < 11; ++k) w[k] = lds_at<uint32_t>(lds, off + 44 * g + 4 * k);
+    auto at2 = [&](int k) { return __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2); };
+    f.d[0] = (uint16_t)(w[0] & 0xffffu);
+    f.qh[0] = at2(0);
+    f.qs[0] = u32x4{at2(1), at2(2), at2(3), at2(4)};
+    f.d[1] = (uint16_t)(w[5] >> 16);
+    f.qh[1] = w[6];
+    f.qs[1] = u32x4{w[7], w[8], w[9], w[10]};
   } else {
     static_assert(KIND == K_IQ4_NL || KIND == K_Q4_0, "the dword types");  // 36 bytes: d, 16 code bytes, twice
     uint32_t w[9];

@@ -12,7 +12,7 @@
 // wave) meet in LDS, one barrier a group and one wave adding them, the waves in turn; two buffers, so that the others
 // go on with the next group meanwhile.
 //
-// Staged rows (Q4_K, Q6_K, Q8_0 rows of a multiple of 16 bytes; kStagedRows). Read straight into registers, a wave's
+// Staged rows (Q4_K, Q6_K, Q8_0, Q4_0, Q5_0 and IQ4_NL rows of a multiple of 16 bytes; kStagedRows). Read straight into registers, a wave's
 // field loads touch the cache lines of 16 rows each and one row group is in flight: the texture units, not HBM, set
 // the pace (lm_head 183 us; staged, and with inexact weights, 111). Staged, a wave's part of a row group comes by contiguous 16-byte direct loads
 // (global_load_lds_dwordx4) into one of its two slabs, and the fields are read from there into registers, after which
@@ -184,7 +184,8 @@ __device__ __forceinline__ void add_step(const RunPair<KIND>& f, const u32x4 (&a
 }
 
 template <int KIND>
-constexpr bool kStagedRows = KIND == K_Q4_K || KIND == K_Q6_K || KIND == K_Q8_0;
+constexpr bool kStagedRows = KIND == K_Q4_K || KIND == K_Q6_K || KIND == K_Q8_0 || KIND == K_IQ4_NL || KIND == K_Q4_0 ||
+                             KIND == K_Q5_0;
 // 16-byte pieces of a wave's part of a row, from the aligned one that holds its first byte (an even one), and the pitch
 template <int KIND, int SPW>
 constexpr int kPieces = (SPW * kStepBytes<KIND>) % 16 == 0 ? SPW * kStepBytes<KIND> / 16
