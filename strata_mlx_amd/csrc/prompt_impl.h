@@ -1087,6 +1087,12 @@ constexpr int kWaves = 4;
 constexpr int kTiles = 3;  // tiles a chunk at most (an expert's rows decoded once for them)
 constexpr bool kStaged = true;  // rows through LDS by direct loads (run_chunk_staged)
 
+// staged rows read whole dwords: the stacks' bases and a row's bytes multiples of 4
+inline bool rows_staged(const PromptParams& p) {
+  return ((uintptr_t)p.blocks[0] & 3) == 0 && ((uintptr_t)p.blocks[1] & 3) == 0 && p.row_bytes % 4 == 0 &&
+         p.mat_bytes % 4 == 0;
+}
+
 template <int KIND, int MODE, typename OT>
 int launch_prompt(PromptParams& p, hipStream_t s) {
   constexpr int rpw = rows_per_wg<MODE>(kWaves);
@@ -1100,9 +1106,7 @@ int launch_prompt(PromptParams& p, hipStream_t s) {
     hipLaunchKernelGGL((prompt_kernel<KIND, MODE, OT, kWaves, kTiles, decltype(staged)::value, decltype(part)::value>),
                        dim3((unsigned)grid), dim3(64 * kWaves), 0, s, p);
   };
-  // staged rows read whole dwords: the stacks' bases and a row's bytes multiples of 4
-  const bool aligned = ((uintptr_t)p.blocks[0] & 3) == 0 && ((uintptr_t)p.blocks[1] & 3) == 0 &&
-                       p.row_bytes % 4 == 0 && p.mat_bytes % 4 == 0;
+  const bool aligned = rows_staged(p);
   // the dword types: whole groups of rows a wave, rows of a slot or more
   const bool whole = p.rows % (MODE == PM_GLU ? 16 : 32) == 0 && p.row_bytes >= 4 * kSlotDwords<KIND>;
   const bool staged = kStaged && kStagedKind<KIND> && aligned && (!kDwordRows<KIND> || whole);

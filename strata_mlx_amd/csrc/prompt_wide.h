@@ -21,7 +21,9 @@
 //
 // Double-buffered decoded steps (2 x 64 KB): a wave decodes step k + 1 into one buffer, then multiplies step k
 // from the other, then meets the others at the step's one barrier, after which both buffers change roles. A wave's
-// own fields are loaded two steps ahead, and the activations of its tiles (16 slots each, read by row index
+// own rows come into its LDS slots by direct loads, a step ahead of their decode (prompt_impl.h's staged rows; where the
+// stacks do not allow them, straight into registers two steps ahead: 8192 tokens of IQ3_S 4565 us, staged 4458), and the
+// activations of its tiles (16 slots each, read by row index
 // straight into MFMA operand registers) one step ahead, each register asked for again once step k's MFMAs have
 // read it.
 //
@@ -160,9 +162,10 @@ __device__ __forceinline__ void wide_decode(const RunPair<KIND>& f, int g, const
 
 // One item: chunk tiles t0 .. t0 + nt - 1 of expert e, row block rb; this wave's NTW tiles (t0 + wave + 4 i). Every
 // wave runs the same steps and barriers whatever its NTW.
-template <int KIND, int MODE, typename OT, int NTW>
+template <int KIND, int MODE, typename OT, int NTW, bool STAGED>
 __device__ __forceinline__ void wide_item(const PromptParams& p, const DirectTables<KIND>& tab, u32x4* wdec,
-                                          float* ratio, float* last, uint32_t e, int t0, int rb, int wave, int lane) {
+                                          float* ratio, float* last, const uint8_t* slots, uint32_t e, int t0, int rb,
+                                          int wave, int lane) {
   const int n = lane & 15, g = lane >> 4;
   constexpr bool kGlu = MODE == PM_GLU;
   // this wave's groups of rows, wave + kWideWaves j: SwiGLU form, the first half of the groups gate rows, the second
@@ -178,6 +181,24 @@ __device__ __forceinline__ void wide_item(const PromptParams& p, const DirectTab
     off[j] = (uint32_t)min(grow, p.rows - 1) * (uint32_t)p.row_bytes;  // past the last row: the last
   }
   const LaneOffsets<KIND> o = strata_mv::lane_offsets<KIND>(g);
+  // STAGED: the wave's dwords of a slot load (its group's row q, dword d), and its slots
+  constexpr int kGL = STAGED ? kGroupLoads<KIND> : 1;
+  uint32_t voff[kGL];
+  const uint32_t slot0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)slots + (uint32_t)(wave * 256 * kGL));
+  if constexpr (STAGED) {
+    static_assert(kGroupsWave == 1, "a group a wave");
+    const int first = kGlu ? rb * 16 * kHalf + 16 * (wave % kHalf) : rb * 16 * kWideGroups + 16 * wave;
+#pragma unroll
+    for (int i = 0; i < kGL; ++i) {
+      const int c = 64 * i + lane, q = c / kSlotPitch<KIND>, d = min(c % kSlotPitch<KIND>, kSlotDwords<KIND> - 1);
+      voff[i] = (uint32_t)min(first + q, p.rows - 1) * (uint32_t)p.row_bytes + 4u * (uint32_t)d;
+    }
+  }
+  auto stage = [&](int k) {
+    const uint8_t* base = mat[0] + ((uint32_t)(k * kStepBytes<KIND>) & ~3u);
+#pragma unroll
+    for (int i = 0; i < kGL; ++i) dma_dword(base, voff[i], slot0 + 256u * i);
+  };
   const int nsteps = p.cols / kStep;
   const uint32_t step_bytes = (uint32_t)(p.row_bytes / nsteps);
 
@@ -201,17 +222,35 @@ __device__ __forceinline__ void wide_item(const PromptParams& p, const DirectTab
       if (k + 1 == nsteps && g == 0) last[gi * 16 + n] = s[j];
     }
   };
+  // STAGED: step k's fields from the slots, in registers when it returns; its loads are waited for by the caller
   auto fields = [&](int k, int slot) {
+    if constexpr (STAGED) {
+      const uint8_t* row = slots + wave * 256 * kGL + 4 * kSlotPitch<KIND> * n;
+      if (k & 1)
+        lds_fields<KIND, 2>(row, g, f[slot][0]);
+      else
+        lds_fields<KIND, 0>(row, g, f[slot][0]);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < kGroupsWave; ++j)
       strata_mv::load_fields<KIND>(mat[j], off[j] + (uint32_t)k * step_bytes, o, f[slot][j]);
   };
 #pragma unroll
   for (int j = 0; j < kGroupsWave; ++j) s[j] = 1.0f;
-  fields(0, 0);
-  fields(nsteps > 1 ? 1 : 0, 1);
-  decode(0, 0);
-  if (nsteps > 2) fields(2, 0);
+  if constexpr (STAGED) {
+    stage(0);
+    wait_loads();
+    fields(0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (nsteps > 1) stage(1);
+    decode(0, 0);
+  } else {
+    fields(0, 0);
+    fields(nsteps > 1 ? 1 : 0, 1);
+    decode(0, 0);
+    if (nsteps > 2) fields(2, 0);
+  }
   lds_barrier();
 
   f32x4 acc[kWideGroups][NTW > 0 ? NTW : 1];
@@ -235,8 +274,16 @@ __device__ __forceinline__ void wide_item(const PromptParams& p, const DirectTab
       const int k = kb + sp;
       if (k < nsteps) {
         if (k + 1 < nsteps) {  // step k + 1 into the other buffer, then its fields' slot takes step k + 3's
-          decode(k + 1, sp ^ 1);
-          if (k + 3 < nsteps) fields(k + 3, sp ^ 1);
+          if constexpr (STAGED) {
+            wait_loads();
+            fields(k + 1, sp ^ 1);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (k + 2 < nsteps) stage(k + 2);
+            decode(k + 1, sp ^ 1);
+          } else {
+            decode(k + 1, sp ^ 1);
+            if (k + 3 < nsteps) fields(k + 3, sp ^ 1);
+          }
         }
         if constexpr (NTW > 0 && has_step_scale<KIND>()) {  // the sums into step k's scale
 #pragma unroll
@@ -306,8 +353,9 @@ __device__ __forceinline__ void wide_item(const PromptParams& p, const DirectTab
   }
 }
 
-template <int KIND, int MODE, typename OT>
+template <int KIND, int MODE, typename OT, bool STAGED>
 __global__ __launch_bounds__(kWideThreads, kWideWavesSimd) void prompt_wide_kernel(PromptParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t slots[STAGED ? kWideWaves * 256 * kGroupLoads<KIND> : 16];
   static_assert(kWideGroups % kWideWaves == 0 && kWideGroups % 2 == 0, "whole groups of rows a wave");
   static_assert(MODE == PM_GLU || MODE == PM_SCATTER, "the SwiGLU and scatter forms");
   __shared__ __attribute__((aligned(16))) u32x4 wdec[2 * kWideBuf];
@@ -331,7 +379,7 @@ __global__ __launch_bounds__(kWideThreads, kWideWavesSimd) void prompt_wide_kern
     const int c = it / p.row_blocks, rb = it % p.row_blocks;
     const int t0 = (int)chunks[c];
     const uint32_t e = p.tile_expert[t0];
-    wide_item<KIND, MODE, OT, kWideTilesWave>(p, tab, wdec, ratio, last, e, t0, rb, wave, lane);  // a full chunk
+    wide_item<KIND, MODE, OT, kWideTilesWave, STAGED>(p, tab, wdec, ratio, last, slots, e, t0, rb, wave, lane);  // a full chunk
   }
 }
 
@@ -354,7 +402,10 @@ int launch_prompt_wide(PromptParams& p, hipStream_t s) {
     p.row_blocks = (p.rows + rows - 1) / rows;
     const int grid = kWidePerCU * strata_mv::device_cus() / kXcds * kXcds;
     if (grid < kXcds) return STRATA_ERR_SHAPE;
-    hipLaunchKernelGGL((prompt_wide_kernel<KIND, MODE, OT>), dim3((unsigned)grid), dim3(kWideThreads), 0, s, p);
+    if (rows_staged(p))
+      hipLaunchKernelGGL((prompt_wide_kernel<KIND, MODE, OT, true>), dim3((unsigned)grid), dim3(kWideThreads), 0, s, p);
+    else
+      hipLaunchKernelGGL((prompt_wide_kernel<KIND, MODE, OT, false>), dim3((unsigned)grid), dim3(kWideThreads), 0, s, p);
     STRATA_CHECK_LAUNCH();
     return STRATA_OK;
   } else {
