@@ -1,5 +1,6 @@
 // One block type's instances of the matvec and dequant kernels. The build compiles this file once per
 // type, with -DSTRATA_KIND=<GGUF type id>, so the types compile in parallel.
+#include "dequant_impl.h"
 #include "direct_impl.h"
 
 #ifndef STRATA_KIND
@@ -18,7 +19,7 @@ int STRATA_CAT(matvec_launch_, STRATA_KIND)(MatvecParams& p, int x_dtype, int ou
 
 int STRATA_CAT(dequant_launch_, STRATA_KIND)(const uint8_t* blocks, int64_t runs_total, int runs_per_row,
                                              int row_bytes, void* out, int out_dtype, hipStream_t s) {
-  return launch_dequant_kind<STRATA_KIND>(blocks, runs_total, runs_per_row, row_bytes, out, out_dtype, s);
+  return launch_dequant_any<STRATA_KIND>(blocks, runs_total, runs_per_row, row_bytes, out, out_dtype, s);
 }
 
 }  // namespace strata_mv
