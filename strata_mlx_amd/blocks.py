@@ -37,8 +37,9 @@ TOKENS_TILE = 16  # slots of a tile (strata_mlx/blocks.py:581)
 # 77 against 57.
 TILES_FROM = 48
 # the same where gate and up take the persistent or codebook decode kernels at 4096 inputs (IQ3_S, Q2_0; IQ3_XXS in
-# float16): IQ3_S 8 tokens 130 us against 137, 9 tokens 171 against 138
-TILES_FROM_DECODE = 65
+# float16): a whole MoE block of IQ3_S, float16: 8 tokens 190 us against 197 in tiles, 9 tokens 298 against 303, 10 tokens
+# 319 against 307
+TILES_FROM_DECODE = 73
 TILES_FROM_ANY = 1600  # what the fused tile kernels do not take (float32, ragged rows)
 MATVEC_GLU_UPTO = 1 << 16  # pairs for which down takes silu(gate) * up itself (the reference: 30)
 

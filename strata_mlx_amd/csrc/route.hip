@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kBlock) void route_place(const uint32_t* idx, int p
 // naming one expert found bit by bit of the expert's number, a ballot each), with a count per wave and expert in LDS;
 // then per expert the waves' exclusive prefix and the tiles; then each pair's slot. Every slot is written once: an
 // expert's empty slots and the unused tiles' by themselves, no pass that clears them all first. Bound by latency, not
-// by work: three launches take 16-20 us at these sizes (their gaps included), this one 6-9 us (384 to 4096 pairs).
+// by work: three launches take 16-20 us at these sizes (their gaps included), this one 10-12 us (3072 pairs).
 constexpr int kSmallPairs = 4096, kSmallExperts = 1024, kSmallWaves = 16;
 constexpr int kSmallChunks = kSmallPairs / (64 * kSmallWaves);  // chunks of 64 pairs a wave at most
 
